@@ -38,6 +38,10 @@
 // eps = 2^-13 ||q||_1 max|k| bounds |s~ - s| for 64 (anchor) or 128 (partner
 // hi + lo) bf16 products summed in fp32 (the bound of rlm_select_tile.hip),
 // with max|k| taken over every key the workgroup scored for the routing.
+//
+// The single-anchor sequence form over longer caches is the S = 1 case (SINGLE):
+// it differs in what a query without a candidate reports, and in the results for
+// scores that are not finite, both as select_kernel's.
 #include "rlm_common.hpp"
 #include "rlm_multi_tile.hpp"
 #include "rlm_tile_util.hpp"
@@ -324,8 +328,8 @@ __device__ __forceinline__ uint32_t key_off(const MultiTileParams& p, int64_t b,
 // selection key (score, tie index) in the member's 4 lanes; when the score is
 // not above -inf, c + 1 instead: below every selection key (whose high word is
 // nonzero) and distinct per member, so such a member ranks last and counts as
-// absent.
-template <bool ANCHOR>
+// absent.  RAW: the selection key of any score.
+template <bool ANCHOR, bool RAW>
 __device__ __forceinline__ uint64_t member_key(const MultiTileParams& p, const MRec& R, int c,
                                                int t, int ls, int sub, const double* qrow,
                                                rsrc_t keys, int64_t b, int s) {
@@ -353,22 +357,35 @@ __device__ __forceinline__ uint64_t member_key(const MultiTileParams& p, const M
   d += dpp_f64<kDppXor1>(d);
   d += dpp_f64<kDppXor2>(d);
   const float score = static_cast<float>(d * p.exact_scale);
-  return score > -INFINITY ? select_key(score, static_cast<uint32_t>(ANCHOR ? pos : c))
-                           : static_cast<uint64_t>(c) + 1;
+  return RAW || score > -INFINITY
+             ? select_key(score, static_cast<uint32_t>(ANCHOR ? pos : c))
+             : static_cast<uint64_t>(c) + 1;
 }
 
-// Writes entry `slot` of output row `orow` from key `key` (high word 0: none).  Anchor:
-// none is anchor 0 with score -inf (multi_relation_blocks.py:94); partner:
-// none is the exhausted entry, position t - L + 1 with score -inf
-// (relation_select.py:298-308).  Returns the position, -1 for none.
-template <bool ANCHOR>
+// Writes entry `slot` of output row `orow` from key `key` (0: none).
+//   anchor   a score above -inf, else position 0 and -inf
+//            (multi_relation_blocks.py:94); SINGLE: any key, else t - L + 1 and -inf
+//   partner  a score above -inf, else the exhausted entry, position t - L + 1
+//            and -inf (relation_select.py:298-308).  SINGLE, when the query's
+//            first key is a NaN (`nan_top`): with at most 256 candidate lanes
+//            every entry is exhausted, with more a NaN's entry keeps its
+//            position, as select_kernel's two rankings have it.
+// Returns the position, -1 for none.
+template <bool ANCHOR, bool SINGLE>
 __device__ __forceinline__ int emit(const MultiTileParams& p, const MRec& R, int64_t orow,
-                                    int slot, uint64_t key, int t, int ls) {
-  int pos = ANCHOR ? 0 : t - p.L + 1;
+                                    int slot, uint64_t key, int t, int ls, bool nan_top) {
+  int pos = ANCHOR && !SINGLE ? 0 : t - p.L + 1;
   float score = -INFINITY;
   int found = -1;
-  if ((key >> 32) != 0) {
-    score = key_score(key);
+  const float ks = key_score(key);
+  bool have = ANCHOR && SINGLE ? key != 0 : ks > -INFINITY;
+  if (!ANCHOR && SINGLE && nan_top) {
+    const bool few = p.CAP <= 4 * kWave;
+    if (few) have = false;
+    else if (key != 0 && ks != ks) have = true;
+  }
+  if (have) {
+    if (ANCHOR || ks > -INFINITY) score = ks;
     const int tie = static_cast<int>(key_index(key));
     if (ANCHOR) {
       pos = tie;
@@ -393,7 +410,7 @@ __device__ __forceinline__ int emit(const MultiTileParams& p, const MRec& R, int
 // else k = K, ties to the lowest candidate lane.  The record's anchors so far
 // (taken[0..nact)) are not candidates.  `qrow` is the float64 query and `qn1` its L1 norm.  Returns the
 // anchor position (ANCHOR; -1 for none).
-template <bool ANCHOR>
+template <bool ANCHOR, bool SINGLE, bool ANY>
 __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int lane,
                             const double* qrow, float qn1, float kmax, rsrc_t keys, int64_t b,
                             int s, int64_t orow) {
@@ -401,6 +418,19 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
   const int t = R.t, ls = R.ls;
   const int K = ANCHOR ? 1 : p.K;
   float* sc = L.sc + qi * (p.q_bytes >> 2);
+  const float eps = kErrScale * qn1 * kmax;
+  // Scores that may not be finite (wave-uniform): the filter's bound does not
+  // hold, so every candidate becomes a member (ANY only).
+  constexpr bool kRaw = ANY && (SINGLE || !ANCHOR);
+  const bool wild = ANY && !(eps <= kErrFinite);
+  if (wild) {
+    for (int c = lane; c < p.CAP; c += kWave) {
+      bool v;
+      cand_pos(p, R, c, t, ls, v);
+      sc[c] = v ? 0.0f : -INFINITY;
+    }
+    wave_sync();
+  }
   // The query's anchors so far are not candidates: lane x < nact puts -inf in
   // the lane of anchor x, if it is a candidate of this routing (local window,
   // else its block's pick).  Anchors are at most t.
@@ -449,8 +479,7 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
     }
     theta = prefix >= 0x00800000u ? key_to_float(prefix) : -INFINITY;  // key of -FLT_MAX
   }
-  const float eps = kErrScale * qn1 * kmax;
-  const float thr = theta - (2.0f * eps + kErrAbs);
+  const float thr = wild ? -INFINITY : theta - (2.0f * eps + kErrAbs);
   // Members (candidates with s~ >= thr) numbered in candidate order; those of
   // window [lo, lo + 64) go to the list (others to its trash entry).
   uint64_t* list = L.list + qi * kMListRow;
@@ -494,7 +523,7 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
       const int m = lane >> 2;
       const bool act = m < members;
       const int c = act ? static_cast<int>(list[m]) : 0;
-      const uint64_t key = member_key<ANCHOR>(p, R, c, t, ls, sub, qrow, keys, b, s);
+      const uint64_t key = member_key<ANCHOR, kRaw>(p, R, c, t, ls, sub, qrow, keys, b, s);
       if (act && sub == 0) list[m] = key;
     }
     wave_sync();
@@ -511,9 +540,10 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
         rank += (f < members && k0 > ke) + (f + 1 < members && k1 > ke);
       }
     }
+    const bool nan_top = SINGLE && wild && __builtin_amdgcn_ballot_w64(key_is_nan(ke)) != 0;
     int mine = -1;
-    if (rank < K) mine = emit<ANCHOR>(p, R, orow, rank, ke, t, ls);
-    if (lane >= members && lane < K) emit<ANCHOR>(p, R, orow, lane, 0, t, ls);
+    if (rank < K) mine = emit<ANCHOR, SINGLE>(p, R, orow, rank, ke, t, ls, nan_top);
+    if (lane >= members && lane < K) emit<ANCHOR, SINGLE>(p, R, orow, lane, 0, t, ls, nan_top);
     if (ANCHOR) anchor = wave_max_i(rank == 0 ? mine : -1);
     wave_sync();
     return anchor;
@@ -532,7 +562,7 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
       const int m = m0 + (lane >> 2);
       const bool act = m < nw;
       const int c = act ? static_cast<int>(list[m]) : 0;
-      const uint64_t key = member_key<ANCHOR>(p, R, c, t, ls, sub, qrow, keys, b, s);
+      const uint64_t key = member_key<ANCHOR, kRaw>(p, R, c, t, ls, sub, qrow, keys, b, s);
       if (act && sub == 0) list[m] = key;
     }
     wave_sync();
@@ -553,8 +583,11 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
     wave_sync();
   }
   const uint64_t* topf = L.top + (cur * kMQ + qi) * kMultiTileMaxK;
-  if (lane < K) emit<ANCHOR>(p, R, orow, lane, lane < ntop ? topf[lane] : 0, t, ls);
-  if (ANCHOR && ntop > 0 && (topf[0] >> 32) != 0) anchor = static_cast<int>(key_index(topf[0]));
+  const bool nan_top = SINGLE && wild && ntop > 0 && key_is_nan(topf[0]);
+  if (lane < K)
+    emit<ANCHOR, SINGLE>(p, R, orow, lane, lane < ntop ? topf[lane] : 0, t, ls, nan_top);
+  if (ANCHOR && ntop > 0 && (SINGLE || (topf[0] >> 32) != 0))
+    anchor = static_cast<int>(key_index(topf[0]));
   wave_sync();
   return anchor;
 }
@@ -580,7 +613,7 @@ __device__ __forceinline__ Union candidate_union(const MultiTileParams& p, const
   const MRec& R = L.qr[lane & 15];
   const bool on = R.on != 0;
   uint32_t nlo = ~static_cast<uint32_t>(on ? R.ls : 1 << 30);  // max of ~ls: min of ls
-  uint32_t hi1 = on ? static_cast<uint32_t>(R.t + 1) : 0u;
+  uint32_t hi1 = on && R.t >= 0 ? static_cast<uint32_t>(R.t + 1) : 0u;
   uint32_t plo = on ? static_cast<uint32_t>(R.picks) : 0u;
   uint32_t phi = on ? static_cast<uint32_t>(R.picks >> 32) : 0u;
   union_step<kDppXor1>(nlo, hi1, plo, phi);
@@ -688,7 +721,13 @@ __device__ __forceinline__ float routing_kmax(const MLds& L) {
   return __uint_as_float(kb << 16) * (1.0f + 1.0f / 1024.0f);
 }
 
-template <typename TS>
+// SINGLE: the single-anchor selection (S = 1) with select_kernel's results: slot
+// 0 is active at every position, a query without a candidate reports position
+// t - L + 1 and still routes its partners, from its query-side row alone.
+// ANY: scores that may not be finite get the per-query kernels' results (the
+// multi-anchor instance for NB % 4 == 0 keeps the filtered results for those,
+// and 1.5% of its time).
+template <typename TS, bool SINGLE, bool ANY>
 __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTileParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const MLds L = carve(p, smem);
@@ -776,14 +815,14 @@ __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTilePa
       const int64_t qrow = query_row(qi, active);
       const int64_t orow = qrow * p.S + s;
       if (!active) continue;
-      if (s > L.qr[qi].t) {  // inactive slot: anchor 0, no partners (multi_relation_blocks.py:84, 94)
+      if (!SINGLE && s > L.qr[qi].t) {  // inactive slot: anchor 0, no partners (multi_relation_blocks.py:84, 94)
         if (lane == 0) {
           p.out_anchor[orow] = 0;
           p.out_anchor_score[orow] = -INFINITY;
         }
         continue;
       }
-      const int anchor = exact_select<true>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax,
+      const int anchor = exact_select<true, SINGLE, ANY>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax,
                                             akeys, b, s, orow);
       if (anchor >= 0 && lane == 0) {
         MRec& R = L.qr[qi];
@@ -810,6 +849,7 @@ __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTilePa
     v[1] = pc[lane];
     v[2] = pb[64 + lane];
     v[3] = pc[64 + lane];
+    if (SINGLE && !on) v[1] = v[3] = from_f32<bf16>(0.0f);  // no anchor: the query-side row
   };
   __syncthreads();  // every wave is done with the anchor side's LDS
   bf16 next_rows[4];
@@ -821,7 +861,7 @@ __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTilePa
       if (s + 1 < p.S) partner_rows(s + 1, next_rows);
       L.eq[wave * kMQRow + lane] = static_cast<double>(to_f32(rows[0]) + to_f32(rows[1]));
       L.rq[wave * kMQRow + lane] = static_cast<double>(to_f32(rows[2]) + to_f32(rows[3]));
-      if (lane == 0) L.qr[wave].on = pactive && s < L.qr[wave].nact ? 1 : 0;
+      if (lane == 0) L.qr[wave].on = pactive && (SINGLE || s < L.qr[wave].nact) ? 1 : 0;
     }
     __syncthreads();  // query rows, statistics; previous slot's lists done
     head_scores(p, L, 1, wave, lane);
@@ -853,7 +893,7 @@ __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTilePa
       const int64_t qrow = query_row(qi, active);
       const int64_t orow = qrow * p.S + s;
       if (L.qr[qi].on) {
-        exact_select<false>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax, pkeys, b, s,
+        exact_select<false, SINGLE, ANY>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax, pkeys, b, s,
                             orow);
       } else if (active) {  // inactive (or anchorless) slot: every entry exhausted
         for (int k = lane; k < p.K; k += kWave) {
@@ -898,23 +938,28 @@ hipError_t multi_tile_launch(const MultiTileParams& p, int stat_dtype, hipStream
   const dim3 block(kMThreads);
   const dim3 grid(static_cast<unsigned>(p.B * p.tiles));
   const size_t lds = static_cast<size_t>(p.lds_total);
-#define RLM_MTILE_CASE(TS_ID, TS)                                                          \
-  if (stat_dtype == TS_ID) {                                                               \
+  const bool any = p.single || (p.NB & 3) != 0;
+#define RLM_MTILE_CASE(TS_ID, TS, SINGLE, ANY)                                             \
+  if (stat_dtype == TS_ID && p.single == SINGLE && any == ANY) {                                         \
     static const hipError_t attr = hipFuncSetAttribute(                                    \
-        reinterpret_cast<const void*>(&multi_tile_kernel<TS>),                             \
+        reinterpret_cast<const void*>(&multi_tile_kernel<TS, SINGLE, ANY>),                     \
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                           \
     if (attr != hipSuccess) {                                                              \
-      set_error("multi_relation_select (tile): cannot reserve LDS: %s",                    \
+      set_error("relation selection (tile): cannot reserve LDS: %s",                       \
                 hipGetErrorString(attr));                                                  \
       return attr;                                                                         \
     }                                                                                      \
-    hipLaunchKernelGGL((multi_tile_kernel<TS>), grid, block, lds, stream, p);              \
-    return launch_status("multi_relation_select (tile)");                                  \
+    hipLaunchKernelGGL((multi_tile_kernel<TS, SINGLE, ANY>), grid, block, lds, stream, p);      \
+    return launch_status("relation selection (tile)");                                     \
   }
-  RLM_MTILE_CASE(RLM_F32, float)
-  RLM_MTILE_CASE(RLM_BF16, bf16)
+  RLM_MTILE_CASE(RLM_F32, float, false, false)
+  RLM_MTILE_CASE(RLM_BF16, bf16, false, false)
+  RLM_MTILE_CASE(RLM_F32, float, false, true)
+  RLM_MTILE_CASE(RLM_BF16, bf16, false, true)
+  RLM_MTILE_CASE(RLM_F32, float, true, true)
+  RLM_MTILE_CASE(RLM_BF16, bf16, true, true)
 #undef RLM_MTILE_CASE
-  set_error("multi_relation_select (tile): unsupported statistics dtype %s",
+  set_error("relation selection (tile): unsupported statistics dtype %s",
             dtype_name(stat_dtype));
   return hipErrorInvalidValue;
 }

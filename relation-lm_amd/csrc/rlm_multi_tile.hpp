@@ -1,6 +1,7 @@
 // Parameters of the matrix-core-filtered routed multi-anchor selection
 // (rlm_multi_tile.hip), the path of multi_relation_select_seq for bf16
-// activations, 64-wide exact and router vectors and any cache length.
+// activations, 64-wide exact and router vectors and any cache length, and of
+// relation_select_packed_seq where the cache does not fit LDS (select_tile_kernel).
 #pragma once
 
 #include "rlm_common.hpp"
@@ -18,6 +19,7 @@ struct MultiTileParams {
   int64_t B, Tq, T;
   int S, NB, BS, BS_log2, L, TOP, K, CAP, H, H_log2, HD, RB;
   int strict;
+  bool single;  // single-anchor selection (S = 1) with select_kernel's results
   double exact_scale, head_scale;
   const void* pos;
   int pos_dtype;

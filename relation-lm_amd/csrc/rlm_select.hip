@@ -1381,7 +1381,7 @@ bool tile_params(const SelectParams& p, const Geometry& g, int act, int stat,
       (g.H & (g.H - 1)) != 0)
     return false;
   if (g.T % 16 != 0 || g.T > kTileMaxRows || static_cast<int64_t>(g.NB) * g.BS != g.T) return false;
-  if (g.NB > 64 || g.NB % 4 != 0 || p.CAP > 256 || p.TOP > kTileMaxTop || p.K < 1 || p.K > kTileMaxK) return false;
+  if (g.NB > 64 || p.CAP > 256 || p.TOP > kTileMaxTop || p.K < 1 || p.K > kTileMaxK) return false;
   if (g.H * g.RB > 512) return false;  // both sides' bias tables staged by one thread each
   tp.B = g.B;
   tp.Tq = g.Tq;
@@ -1430,6 +1430,82 @@ bool tile_params(const SelectParams& p, const Geometry& g, int act, int stat,
   tp.out_partner_score = p.out_partner_score;
   tp.tiles = static_cast<int>((g.Tq + 15) / 16);
   return select_tile_layout(tp);
+}
+
+// The multi-anchor selection takes the matrix-core-filtered kernel where it
+// applies unless RLM_MULTI_TILE=0 (both kernels give identical results; the
+// switch exists for comparisons).
+bool multi_tile_path_enabled() {
+  static const bool on = [] {
+    const char* v = std::getenv("RLM_MULTI_TILE");
+    return v == nullptr || v[0] != '0';
+  }();
+  return on;
+}
+
+// Fills the multi-anchor tile kernel's parameters when the shapes fit it:
+// bf16 activations, 64-wide exact and router vectors, whole blocks of at least
+// 16 rows, at most 64 blocks and 1024 candidates.  S = 1 also serves the
+// single-anchor sequence form.
+bool multi_tile_params(const SelectParams& p, int S, const Geometry& g, int act, int stat,
+                       const rlm_tensor* positions, MultiTileParams& tp) {
+  if (act != RLM_BF16 || (stat != RLM_F32 && stat != RLM_BF16)) return false;
+  if (g.E != 64 || g.H * g.HD != 64 || g.H > kMultiTileMaxHeads || g.HD % 4 != 0 ||
+      (g.H & (g.H - 1)) != 0)
+    return false;
+  if (static_cast<int64_t>(g.NB) * g.BS != g.T || g.BS < 16 || g.BS % 16 != 0) return false;
+  if (g.NB > kMultiTileMaxBlocks) return false;
+  if (p.CAP > kMultiTileMaxCap || p.TOP > kMultiTileMaxTop || p.K < 1 || p.K > kMultiTileMaxK)
+    return false;
+  if (S > kMultiTileMaxSlots || g.H * g.RB > 512) return false;
+  tp.B = g.B;
+  tp.Tq = g.Tq;
+  tp.T = g.T;
+  tp.S = S;
+  tp.NB = g.NB;
+  tp.BS = g.BS;
+  tp.BS_log2 = p.BS_log2;
+  tp.L = p.L;
+  tp.TOP = p.TOP;
+  tp.K = p.K;
+  tp.CAP = p.CAP;
+  tp.H = g.H;
+  tp.H_log2 = p.H_log2;
+  tp.HD = g.HD;
+  tp.RB = g.RB;
+  tp.strict = p.strict;
+  tp.exact_scale = p.exact_scale;
+  tp.head_scale = p.head_scale;
+  tp.pos = positions->data;
+  tp.pos_dtype = positions->dtype;
+  tp.pos_sb = p.pos_sb;
+  tp.pos_sq = p.pos_sq;
+  tp.pos_count = p.pos_sb == 0 ? g.Tq : g.B * g.Tq;
+  tp.aq = static_cast<const bf16*>(p.aq);
+  tp.arq = static_cast<const bf16*>(p.arq);
+  tp.pbase = static_cast<const bf16*>(p.pq);
+  tp.pcache = static_cast<const bf16*>(p.pcache);
+  tp.akeys = static_cast<const bf16*>(p.as.keys);
+  tp.pkeys = static_cast<const bf16*>(p.ps.keys);
+  tp.key_bytes = p.key_bytes;
+  tp.amean = p.as.mean;
+  tp.astd = p.as.stdev;
+  tp.pmean = p.ps.mean;
+  tp.pstd = p.ps.stdev;
+  tp.agamma = p.as.gamma;
+  tp.pgamma = p.ps.gamma;
+  tp.abias = p.as.bias;
+  tp.pbias = p.ps.bias;
+  tp.agamma_dtype = p.as.gamma_dtype;
+  tp.pgamma_dtype = p.ps.gamma_dtype;
+  tp.abias_dtype = p.as.bias_dtype;
+  tp.pbias_dtype = p.ps.bias_dtype;
+  tp.out_anchor = p.out_anchor;
+  tp.out_anchor_score = p.out_anchor_score;
+  tp.out_partner = p.out_partner;
+  tp.out_partner_score = p.out_partner_score;
+  tp.tiles = static_cast<int>((g.Tq + 15) / 16);
+  return multi_tile_layout(tp);
 }
 
 // The decode form takes the latency-oriented kernel where it applies unless
@@ -1670,7 +1746,9 @@ hipError_t select_packed_impl(
   p.out_partner_score = static_cast<float*>(out_partner_score->data);
   if (seq && !ring && tile_path_enabled()) {
     // bf16 activations, 64-wide exact and router vectors, caches of at most 512
-    // rows: the matrix-core-filtered kernel (rlm_select_tile.hip).
+    // rows in at most 64 blocks: the matrix-core-filtered kernel
+    // (rlm_select_tile.hip).  B=8, T=448 in 14 blocks: 20 us less than
+    // select_kernel and the projection's own launch.
     TileParams tp{};
     if (tile_params(p, g, act, stat, position, anchor_query, anchor_router_query,
                     partner_base, partner_anchor_cache, anchor_keys, partner_keys,
@@ -1696,6 +1774,18 @@ hipError_t select_packed_impl(
       }
       const hipError_t te = select_tile_launch(tp, stat, stream);
       if (te != hipSuccess || xseq == nullptr || fused) return te;
+      return expand_seq_linear(*xseq, g, stream);
+    }
+    // Longer caches (their rows do not fit LDS) and more than 256 candidates:
+    // the multi-anchor tile kernel with one slot, which reads the candidate
+    // tiles from L2 instead of staging the cache.  B=8, T=2048, block 64, local
+    // 128, top 4, K=8: 131 us, where select_kernel takes 364 us (one float64 dot
+    // per candidate per query).
+    MultiTileParams mp{};
+    if (multi_tile_params(p, 1, g, act, stat, position, mp)) {
+      mp.single = true;
+      const hipError_t me = multi_tile_launch(mp, stat, stream);
+      if (me != hipSuccess || xseq == nullptr) return me;
       return expand_seq_linear(*xseq, g, stream);
     }
   }
@@ -1734,81 +1824,6 @@ bool check_slot_rows(const rlm_tensor* t, const char* name, int64_t d0, int64_t 
                      int64_t width, int act) {
   return check_tensor(t, name, 4) && check_dim(t, name, 0, d0) && check_dim(t, name, 1, d1) &&
          check_dim(t, name, 2, S) && check_dim(t, name, 3, width) && check_dtype_is(t, name, act);
-}
-
-// The multi-anchor selection takes the matrix-core-filtered kernel where it
-// applies unless RLM_MULTI_TILE=0 (both kernels give identical results; the
-// switch exists for comparisons).
-bool multi_tile_path_enabled() {
-  static const bool on = [] {
-    const char* v = std::getenv("RLM_MULTI_TILE");
-    return v == nullptr || v[0] != '0';
-  }();
-  return on;
-}
-
-// Fills the multi-anchor tile kernel's parameters when the shapes fit it:
-// bf16 activations, 64-wide exact and router vectors, whole blocks of at least
-// 16 rows, at most 64 blocks and 1024 candidates.
-bool multi_tile_params(const SelectParams& p, const MultiParams& m, const Geometry& g, int act,
-                       int stat, const rlm_tensor* positions, MultiTileParams& tp) {
-  if (act != RLM_BF16 || (stat != RLM_F32 && stat != RLM_BF16)) return false;
-  if (g.E != 64 || g.H * g.HD != 64 || g.H > kMultiTileMaxHeads || g.HD % 4 != 0 ||
-      (g.H & (g.H - 1)) != 0)
-    return false;
-  if (static_cast<int64_t>(g.NB) * g.BS != g.T || g.BS < 16 || g.BS % 16 != 0) return false;
-  if (g.NB > kMultiTileMaxBlocks || g.NB % 4 != 0) return false;
-  if (p.CAP > kMultiTileMaxCap || p.TOP > kMultiTileMaxTop || p.K < 1 || p.K > kMultiTileMaxK)
-    return false;
-  if (m.S > kMultiTileMaxSlots || g.H * g.RB > 512) return false;
-  tp.B = g.B;
-  tp.Tq = g.Tq;
-  tp.T = g.T;
-  tp.S = m.S;
-  tp.NB = g.NB;
-  tp.BS = g.BS;
-  tp.BS_log2 = p.BS_log2;
-  tp.L = p.L;
-  tp.TOP = p.TOP;
-  tp.K = p.K;
-  tp.CAP = p.CAP;
-  tp.H = g.H;
-  tp.H_log2 = p.H_log2;
-  tp.HD = g.HD;
-  tp.RB = g.RB;
-  tp.strict = p.strict;
-  tp.exact_scale = p.exact_scale;
-  tp.head_scale = p.head_scale;
-  tp.pos = positions->data;
-  tp.pos_dtype = positions->dtype;
-  tp.pos_sb = p.pos_sb;
-  tp.pos_sq = p.pos_sq;
-  tp.pos_count = p.pos_sb == 0 ? g.Tq : g.B * g.Tq;
-  tp.aq = static_cast<const bf16*>(p.aq);
-  tp.arq = static_cast<const bf16*>(p.arq);
-  tp.pbase = static_cast<const bf16*>(p.pq);
-  tp.pcache = static_cast<const bf16*>(p.pcache);
-  tp.akeys = static_cast<const bf16*>(p.as.keys);
-  tp.pkeys = static_cast<const bf16*>(p.ps.keys);
-  tp.key_bytes = p.key_bytes;
-  tp.amean = p.as.mean;
-  tp.astd = p.as.stdev;
-  tp.pmean = p.ps.mean;
-  tp.pstd = p.ps.stdev;
-  tp.agamma = p.as.gamma;
-  tp.pgamma = p.ps.gamma;
-  tp.abias = p.as.bias;
-  tp.pbias = p.ps.bias;
-  tp.agamma_dtype = p.as.gamma_dtype;
-  tp.pgamma_dtype = p.ps.gamma_dtype;
-  tp.abias_dtype = p.as.bias_dtype;
-  tp.pbias_dtype = p.ps.bias_dtype;
-  tp.out_anchor = p.out_anchor;
-  tp.out_anchor_score = p.out_anchor_score;
-  tp.out_partner = p.out_partner;
-  tp.out_partner_score = p.out_partner_score;
-  tp.tiles = static_cast<int>((g.Tq + 15) / 16);
-  return multi_tile_layout(tp);
 }
 
 hipError_t multi_select_impl(
@@ -1931,7 +1946,7 @@ hipError_t multi_select_impl(
   if (queries == 0) return hipSuccess;
   if (multi_tile_path_enabled()) {
     MultiTileParams tp{};
-    if (multi_tile_params(p, m, g, act, stat, positions, tp))
+    if (multi_tile_params(p, m.S, g, act, stat, positions, tp))
       return multi_tile_launch(tp, stat, stream);
   }
   const dim3 block(p.W * kWave);

@@ -76,7 +76,7 @@ struct Lds {
   double* rq;           // [16][kQRow]: router query, float64
   double* eq;           // [16][kQRow]: exact query, float64
   double* sh;           // [H][16][NB]: per-head block scores (aliases `list`)
-  uint64_t* blk;        // [16][NB]: block selection keys
+  uint64_t* blk;        // [16][NBP]: block selection keys, padded to an even count with 0
   uint64_t* list;       // [16][kListCap]
   uint64_t* top;        // [2][16][kTileMaxK]
   uint16_t* frag;       // [hi, lo][16][64] bf16 partner query (aliases `top`)
@@ -291,8 +291,8 @@ __device__ void head_scores(const TileParams& p, const Lds& L, int side, int wav
   }
 }
 
-// Block picks of all 16 queries, one lane per (query, block): pair g = 16 NB
-// pairs in query order on waves [0, NB / 4) (NB % 4 == 0).
+// Block picks of all 16 queries, one lane per (query, block): the 16 NB pairs in
+// query order on the first waves.
 //   block_keys: the log-sum-exp over the H heads (relation_select.py:97-106)
 //     of the per-head scores, summed as the pairwise tree ((e0 + e1) + (e2 +
 //     e3)) + ..., and the 64-bit selection key (score, lower block first) of
@@ -302,7 +302,10 @@ __device__ void head_scores(const TileParams& p, const Lds& L, int side, int wav
 //     (:229-242) -- into the query's candidate table.
 // Each query's wave clears its table first (picks past the last block are
 // block 0, invalid) and sets the local-window entry.
-template <int HL>
+// Keys per query in `blk`: even, so that a row's keys are read two at a time.
+__host__ __device__ __forceinline__ int blk_stride(const TileParams& p) { return (p.NB + 1) & ~1; }
+
+template <int HL, bool ANY>
 __device__ __forceinline__ void block_keys(const TileParams& p, const Lds& L, int g) {
   constexpr int H = 1 << HL;
   const int q = g / p.NB;
@@ -325,13 +328,16 @@ __device__ __forceinline__ void block_keys(const TileParams& p, const Lds& L, in
   const int ls = t - p.L + 1 > 0 ? t - p.L + 1 : 0;
   const int end = (j + 1) * p.BS - 1;
   const bool eligible = end <= t && (!p.strict || end < ls);
-  L.blk[g] = select_key(eligible ? static_cast<float>(lse) : -INFINITY, static_cast<uint32_t>(j));
+  uint64_t* row = L.blk + q * (ANY ? blk_stride(p) : p.NB);
+  row[j] = select_key(eligible ? static_cast<float>(lse) : -INFINITY, static_cast<uint32_t>(j));
+  if (ANY && j == p.NB - 1 && (p.NB & 1)) row[p.NB] = 0;  // the pad: below every key
 }
 
+template <bool ANY>
 __device__ __forceinline__ void block_ranks(const TileParams& p, const Lds& L, int g) {
   const int q = g / p.NB;
   const int j = g - q * p.NB;
-  const uint64_t* row = L.blk + q * p.NB;
+  const uint64_t* row = L.blk + q * (ANY ? blk_stride(p) : p.NB);
   const uint64_t kj = row[j];
   int rank = 0;
   for (int k = 0; k < p.NB; k += 2) {
@@ -349,15 +355,16 @@ __device__ __forceinline__ void block_ranks(const TileParams& p, const Lds& L, i
 
 // The picks phase of one stream, between two workgroup barriers: keys, then
 // (once every key of a query is written) ranks.
+template <bool ANY>
 __device__ __forceinline__ void block_picks(const TileParams& p, const Lds& L, int wave, int lane) {
   const int g = wave * kWave + lane;
-  const bool mine = g < kQ * p.NB;  // whole waves: 16 NB is a multiple of 64
+  const bool mine = g < kQ * p.NB;
   if (mine) {
     switch (p.H_log2) {
-      case 0: block_keys<0>(p, L, g); break;
-      case 1: block_keys<1>(p, L, g); break;
-      case 2: block_keys<2>(p, L, g); break;
-      default: block_keys<3>(p, L, g); break;
+      case 0: block_keys<0, ANY>(p, L, g); break;
+      case 1: block_keys<1, ANY>(p, L, g); break;
+      case 2: block_keys<2, ANY>(p, L, g); break;
+      default: block_keys<3, ANY>(p, L, g); break;
     }
   }
   // A query's keys sit in one wave when NB divides 64, else they may span two.
@@ -366,7 +373,7 @@ __device__ __forceinline__ void block_picks(const TileParams& p, const Lds& L, i
   } else {
     wave_sync();
   }
-  if (mine) block_ranks(p, L, g);
+  if (mine) block_ranks<ANY>(p, L, g);
 }
 
 // Clears the wave's query's candidate table: the local window (positions
@@ -432,12 +439,15 @@ __device__ __forceinline__ uint64_t member_key(const TileParams& p, const Lds& L
 
 // Output slot `slot` of the wave's query from the 64-bit key `key` or, when
 // !have, the exhausted-slot sentinel (position t - L + 1, score -inf;
-// relation_select.py:298-308).  Returns the position.
+// relation_select.py:298-308).  `wild`: a partner key not above -inf counts as
+// exhausted.  Returns the position.
 template <bool ANCHOR>
 __device__ __forceinline__ int emit(const TileParams& p, const QRec& R, int64_t qrow, int slot,
-                                    bool have, uint64_t key, int t, int ls, bool active) {
+                                    bool have, uint64_t key, int t, int ls, bool active,
+                                    bool wild) {
   int pos = t - p.L + 1;
   float score = -INFINITY;
+  if (!ANCHOR && wild) have = have && key_score(key) > -INFINITY;
   if (have) {
     score = key_score(key);
     const int tie = static_cast<int>(key_index(key));
@@ -464,7 +474,7 @@ __device__ __forceinline__ int emit(const TileParams& p, const QRec& R, int64_t 
 // query qi, written to the outputs.  ANCHOR: k = 1, ties to the lowest position
 // (returns the anchor); else k = p.K, ties to the lowest candidate lane, and
 // `exclude` is not a candidate.  `qrow` is the float64 query, `qn1` its L1 norm.
-template <bool ANCHOR>
+template <bool ANCHOR, bool ANY>
 __device__ int exact_select(const TileParams& p, const Lds& L, int qi, int lane, int t, int ls,
                             int exclude, const double* qrow, float qn1, float kmax, bool active,
                             int64_t qrow_out) {
@@ -519,11 +529,15 @@ __device__ int exact_select(const TileParams& p, const Lds& L, int qi, int lane,
     theta = prefix >= 0x00800000u ? key_to_float(prefix) : -INFINITY;  // key of -FLT_MAX
   }
   const float eps = kErrScale * qn1 * kmax;
+  // Scores that may not be finite (wave-uniform): the filter's bound does not
+  // hold, so every candidate becomes a member, and the list is what
+  // select_kernel gives for such scores (ANY only).
+  const bool wild = ANY && !(eps <= kErrFinite);
   const float thr = theta - (2.0f * eps + kErrAbs);
   uint32_t mask = 0;
 #pragma unroll
   for (int i = 0; i < kMaxNCL; ++i)
-    if (st[i] > -INFINITY && st[i] >= thr) mask |= 1u << i;
+    if (wild ? ok[i] : st[i] > -INFINITY && st[i] >= thr) mask |= 1u << i;
   int mi[kMaxNCL];
   const int members = number_members<kMaxNCL>(mask, mi);
   uint64_t* list = L.list + qi * kListCap;
@@ -558,8 +572,10 @@ __device__ int exact_select(const TileParams& p, const Lds& L, int qi, int lane,
       }
     }
     int mine = -(1 << 30) - 1;
-    if (rank < K) mine = emit<ANCHOR>(p, R, qrow_out, rank, true, ke, t, ls, active);
-    if (lane >= members && lane < K) emit<ANCHOR>(p, R, qrow_out, lane, false, 0, t, ls, active);
+    // A NaN (clear sign bit: above every number) as the first key ends the list.
+    const bool ended = !ANCHOR && wild && __builtin_amdgcn_ballot_w64(key_is_nan(ke)) != 0;
+    if (rank < K) mine = emit<ANCHOR>(p, R, qrow_out, rank, !ended, ke, t, ls, active, wild);
+    if (lane >= members && lane < K) emit<ANCHOR>(p, R, qrow_out, lane, false, 0, t, ls, active, wild);
     if (ANCHOR && members > 0) anchor = wave_max_i(rank == 0 ? mine : -(1 << 30) - 1);
     wave_sync();
     return anchor;
@@ -604,7 +620,8 @@ __device__ int exact_select(const TileParams& p, const Lds& L, int qi, int lane,
   const uint64_t* topf = L.top + (cur * kQ + qi) * kTileMaxK;
   if (lane < K) {
     const uint64_t key = lane < ntop ? topf[lane] : 0;
-    emit<ANCHOR>(p, R, qrow_out, lane, lane < ntop, key, t, ls, active);
+    const bool ended = !ANCHOR && wild && ntop > 0 && key_is_nan(topf[0]);
+    emit<ANCHOR>(p, R, qrow_out, lane, lane < ntop && !ended, key, t, ls, active, wild);
   }
   if (ANCHOR && ntop > 0) anchor = static_cast<int>(key_index(topf[0]));
   wave_sync();
@@ -760,7 +777,10 @@ __device__ void expand_rest(const TileParams& p, unsigned char* stage, int64_t w
 }
 
 // XP: the launch also projects the expanded cache (TileParams::x_*).
-template <typename TS, bool XP>
+// ANY: any number of blocks up to 64, and for scores that may not be finite the
+// per-query kernel's results (the instance for NB % 4 == 0 keeps the filtered
+// results for those, and 1% of its time).
+template <typename TS, bool XP, bool ANY>
 __global__ void __launch_bounds__(kThreads) select_tile_kernel(const TileParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Lds L = carve(p, smem);
@@ -861,9 +881,9 @@ __global__ void __launch_bounds__(kThreads) select_tile_kernel(const TileParams 
   }
   __syncthreads();  // B1: s~ and the head scores complete
 
-  block_picks(p, L, wave, lane);
+  block_picks<ANY>(p, L, wave, lane);
   __syncthreads();  // every query's picks are in its candidate table
-  const int anchor = exact_select<true>(p, L, qi, lane, t, ls, -1, L.eq + qi * kQRow, qn1, kmax,
+  const int anchor = exact_select<true, ANY>(p, L, qi, lane, t, ls, -1, L.eq + qi * kQRow, qn1, kmax,
                                         active, qrow);
   clear_table(p, L, qi, lane, t);
 
@@ -930,9 +950,9 @@ __global__ void __launch_bounds__(kThreads) select_tile_kernel(const TileParams 
   }
   __syncthreads();  // B4: s~ and the head scores complete
 
-  block_picks(p, L, wave, lane);
+  block_picks<ANY>(p, L, wave, lane);
   __syncthreads();  // every query's picks are in its candidate table
-  exact_select<false>(p, L, qi, lane, t, ls, anchor, L.eq + qi * kQRow, qn1, kmax, active, qrow);
+  exact_select<false, ANY>(p, L, qi, lane, t, ls, anchor, L.eq + qi * kQRow, qn1, kmax, active, qrow);
 }
 
 }  // namespace
@@ -952,7 +972,7 @@ bool select_tile_layout(TileParams& p) {
   const int list_bytes = kQ * kListCap * 8;
   const int sh_bytes = p.H * kQ * p.NB * 8;
   p.off_list = take(list_bytes > sh_bytes ? list_bytes : sh_bytes);  // per-head scores alias the lists
-  p.off_blk = take(kQ * p.NB * 8);
+  p.off_blk = take(kQ * blk_stride(p) * 8);
   p.off_lmax = 0;
   p.off_top = take(2 * kQ * kTileMaxK * 8);
   p.off_qrec = take(kQ * static_cast<int>(sizeof(QRec)));
@@ -969,22 +989,26 @@ hipError_t select_tile_launch(const TileParams& p, int stat_dtype, hipStream_t s
   const size_t lds = static_cast<size_t>(p.lds_total);
   // The LDS opt-in above 64 KiB is a per-process function attribute (set once
   // per instantiation, for the full 160 KiB).
-#define RLM_TILE_CASE(TS_ID, TS, XP)                                                      \
-  if (stat_dtype == TS_ID && (p.x_out != nullptr) == XP) {                                \
+#define RLM_TILE_CASE(TS_ID, TS, XP, ANY)                                                 \
+  if (stat_dtype == TS_ID && (p.x_out != nullptr) == XP && ((p.NB & 3) != 0) == ANY) {                                \
     static const hipError_t attr = hipFuncSetAttribute(                                   \
-        reinterpret_cast<const void*>(&select_tile_kernel<TS, XP>),                       \
+        reinterpret_cast<const void*>(&select_tile_kernel<TS, XP, ANY>),                       \
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                          \
     if (attr != hipSuccess) {                                                             \
       set_error("relation_select (tile): cannot reserve LDS: %s", hipGetErrorString(attr)); \
       return attr;                                                                        \
     }                                                                                     \
-    hipLaunchKernelGGL((select_tile_kernel<TS, XP>), grid, block, lds, stream, p);        \
+    hipLaunchKernelGGL((select_tile_kernel<TS, XP, ANY>), grid, block, lds, stream, p);        \
     return launch_status("relation_select (tile)");                                       \
   }
-  RLM_TILE_CASE(RLM_F32, float, false)
-  RLM_TILE_CASE(RLM_BF16, bf16, false)
-  RLM_TILE_CASE(RLM_F32, float, true)
-  RLM_TILE_CASE(RLM_BF16, bf16, true)
+  RLM_TILE_CASE(RLM_F32, float, false, false)
+  RLM_TILE_CASE(RLM_BF16, bf16, false, false)
+  RLM_TILE_CASE(RLM_F32, float, true, false)
+  RLM_TILE_CASE(RLM_BF16, bf16, true, false)
+  RLM_TILE_CASE(RLM_F32, float, false, true)
+  RLM_TILE_CASE(RLM_BF16, bf16, false, true)
+  RLM_TILE_CASE(RLM_F32, float, true, true)
+  RLM_TILE_CASE(RLM_BF16, bf16, true, true)
 #undef RLM_TILE_CASE
   set_error("relation_select (tile): unsupported statistics dtype %s", dtype_name(stat_dtype));
   return hipErrorInvalidValue;

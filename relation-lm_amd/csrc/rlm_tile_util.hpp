@@ -103,6 +103,15 @@ __device__ __forceinline__ void load_stat8<bf16>(const bf16* src, float (&out)[8
   }
 }
 
+// The filter's bound holds while scores are finite in fp32: below this eps
+// (||q||_1 max|k| < 2^113).  Above it, or with a NaN, every candidate is verified.
+constexpr float kErrFinite = 1.2676506002282294e30f;  // 2^100
+
+// Whether a key is that of a NaN with a clear sign bit (above every number's).
+__device__ __forceinline__ bool key_is_nan(uint64_t key) {
+  return static_cast<uint32_t>(key >> 32) > 0xff800000u;
+}
+
 // Member indices of the candidates flagged in `mask` (bit i: candidate
 // lane + 64 i), numbered candidate slot by slot; returns the member count.
 template <int NCL>
