@@ -9,11 +9,13 @@
 // it is staged, so the MFMA sees the same operand a bf16 F.linear would.
 //
 //   dma_tile_kernel (M > 64, A of the weight's 16-bit type, K % 64 == 0)
-//                 256x256 workgroup tiles of eight waves (128x128 of four
-//                 waves, two workgroups per CU, for problems under one tile
-//                 per CU) on v_mfma_f32_32x32x16; A and W k-slices of 64 go
+//                 256x256 workgroup tiles of eight waves (128x128 or 64x64 of
+//                 four waves, several workgroups per CU, for problems under one
+//                 tile per CU) on v_mfma_f32_32x32x16; A and W k-slices of 64 go
 //                 from global memory straight into LDS (two stages), the
 //                 output is restaged through LDS into whole row segments.
+//   split_kernel  (M > 64, fp32 A, few tiles) 32x32 tiles, the eight waves of a
+//                 workgroup split K, each through LDS stages of its own.
 //   tile_kernel   (M > 64, the other cases: fp32 A, K % 64 != 0)
 //                 BMxBN workgroup tile (128x128 or 64x128), four
 //                 waves in 2x2, each a (BM/2)x(BN/2) grid of 16x16 MFMA tiles.
@@ -22,8 +24,11 @@
 //                 on the matrix cores.  Workgroups are renumbered so that the
 //                 tiles sharing an A row-block run on the same XCD (one L2),
 //                 which keeps A's HBM traffic at one read.
-//   smallk_kernel (M > 64, K in {32, 64, 96, 128})  e.g. the expanded-cache
-//                 projection (K = relation dim).  A workgroup loads its 128-row
+//   smallk_stream_kernel (M > 64, K in {32, 64, 96, 128}, 16-bit A and W, N a
+//                 multiple of 128)  the expanded-cache projection (K = relation
+//                 dim): W fragments in registers, 64-row A tiles by LDS-DMA.
+//   smallk_kernel (M > 64, K in {32, 64, 96, 128}, the other cases)  A
+//                 workgroup loads its 128-row
 //                 A and W tiles for the whole K once, in one round of
 //                 branch-free buffer loads, into swizzled LDS; each wave then
 //                 forms a 64x64 output tile as (W . A^T) so that a lane holds
@@ -35,10 +40,11 @@
 //                 from global memory in MFMA operand layout, and the partial
 //                 tiles meet once in LDS.
 //
-// fp32 weights: f32_tile_kernel, 64x64 tiles on v_mfma_f32_16x16x4f32 (fp32
-// operands, fp32 accumulation), and f32_skinny_kernel (M <= 64: fp32 FMA dot
-// products split over a wave), so fp32 mode never passes through reduced
-// precision.
+// fp32 weights (fp32 operands and accumulation throughout, so fp32 mode never
+// passes through reduced precision): split_kernel for few tiles and
+// dma_tile_kernel with 64x64 tiles otherwise, both on v_mfma_f32_32x32x2f32;
+// f32_skinny_kernel (M <= 32: fp32 FMA dot products split over a wave); and
+// f32_tile_kernel (v_mfma_f32_16x16x4f32) for K % 32 != 0 or unaligned rows.
 #include "rlm_common.hpp"
 
 namespace rlm {
@@ -742,6 +748,18 @@ __device__ __forceinline__ f32x16 mfma32<f16>(const u16x8& a, const u16x8& b, co
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
+// fp32 operands: the 16 bytes are four consecutive k of the lane's row, one
+// 32x32x2 product each (lane half h of product e holds k = 8 g + 4 h + e of
+// group g; A and W agree on it).
+template <>
+__device__ __forceinline__ f32x16 mfma32<float>(const u16x8& a, const u16x8& b, const f32x16& c) {
+  const f32x4 x = __builtin_bit_cast(f32x4, a), y = __builtin_bit_cast(f32x4, b);
+  f32x16 d = c;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], d, 0, 0, 0);
+  return d;
+}
+
 // Piece swizzle of tile row r (only r % 16 matters) for BK-wide rows.
 template <int BK>
 __device__ __forceinline__ int dma_swz(int r) {
@@ -834,6 +852,8 @@ __device__ __forceinline__ void dma_stage_bias(const GemmParams& p, float* bias_
   }
 }
 
+// W float: the kernel sees fp32 rows as twice as many 16-bit elements (K and lda
+// come doubled), a 16-byte fragment being four fp32 values.
 template <typename W, typename TO, int BM, int BN, int WM, int WN, int NS, int BK>
 __global__ void __launch_bounds__(WM * WN * kWave) dma_tile_kernel(const GemmParams p) {
   constexpr int kWaves = WM * WN;
@@ -974,6 +994,313 @@ __global__ void __launch_bounds__(WM * WN * kWave) dma_tile_kernel(const GemmPar
 }
 
 // ---------------------------------------------------------------------------
+// fp32 A, few output tiles: the waves of a workgroup split K
+// ---------------------------------------------------------------------------
+//
+// Decode batches (64 < M <= a few hundred rows of an fp32 hidden against a
+// 16-bit weight) and small fp32 problems have too few large tiles to fill the
+// chip, and a tile's K loop is then one long chain of load round trips (M = 192,
+// N = 576, K = 2304: 15 tiles of 64 x 128, 42 us).  Here a workgroup of eight
+// waves owns one 32 x 32 output tile and each wave takes every eighth 32-wide
+// chunk of K through its own LDS stages: LDS-DMA moves whole row segments (one
+// L1 access per 128-byte line; fragments loaded straight from global memory
+// touch a line per lane pair, and the L1 then takes 15 us on the shape above),
+// NS chunks in flight per wave, no barrier before the end.  The eight partial
+// tiles meet once in LDS and are added in wave order.  The product is W . A^T,
+// so a lane ends with four consecutive columns of a row.
+constexpr int kSplitWaves = 8;
+
+template <typename W>
+struct SplitForm {
+  static constexpr int kWRow = 32 * static_cast<int>(sizeof(W));  // bytes of a W chunk row
+  static constexpr int kStage = 32 * 128 + 32 * kWRow;            // A and W of one chunk
+  static constexpr int kLoads = kStage / 1024;                    // DMA instructions per chunk
+  static constexpr int NS = sizeof(W) == 2 ? 3 : 2;               // stages per wave
+  static constexpr size_t kLds = static_cast<size_t>(kSplitWaves) * NS * kStage;
+};
+
+template <typename W, typename TO>
+__global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmParams p) {
+  using F = SplitForm<W>;
+  constexpr int NS = F::NS;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int64_t tiles_n = (p.N + 31) / 32;
+  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t m0 = (tile / tiles_n) * 32;
+  const int64_t n0 = (tile % tiles_n) * 32;
+  const rsrc_t ar = make_rsrc(p.a, p.a_bytes);
+  const rsrc_t wr = make_rsrc(p.w, p.w_bytes);
+  unsigned char* mine = smem + wave * (NS * F::kStage);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>(mine)));
+
+  // DMA lane roles.  128-byte rows: eight lanes per row, LDS piece q of row r
+  // holds piece q ^ dma_swz<64>(r); 64-byte rows: four, dma_swz<32>.  Rows past
+  // M or N read zeros.
+  uint32_t a_off[4], w_off[F::kWRow / 32];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int r = 8 * d + (lane >> 3);
+    a_off[d] = m0 + r < p.M ? static_cast<uint32_t>((m0 + r) * p.lda * 4) +
+                                  ((lane & 7) ^ dma_swz<64>(r & 15)) * 16u
+                            : kNoOffset;
+  }
+#pragma unroll
+  for (int d = 0; d < F::kWRow / 32; ++d) {
+    constexpr bool wide = sizeof(W) == 4;
+    const int r = wide ? 8 * d + (lane >> 3) : 16 * d + (lane >> 2);
+    const int q = wide ? (lane & 7) ^ dma_swz<64>(r & 15) : (lane & 3) ^ dma_swz<32>(r & 15);
+    w_off[d] = n0 + r < p.N ? static_cast<uint32_t>((n0 + r) * p.K) * static_cast<uint32_t>(sizeof(W)) + q * 16u
+                            : kNoOffset;
+  }
+  auto issue = [&](int stage, int chunk) {
+    const uint32_t st = lds0 + stage * F::kStage;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      lds_dma16(ar, st + 1024u * d, a_off[d], static_cast<uint32_t>(chunk) * 128u);
+#pragma unroll
+    for (int d = 0; d < F::kWRow / 32; ++d)
+      lds_dma16(wr, st + 4096u + 1024u * d, w_off[d], static_cast<uint32_t>(chunk) * F::kWRow);
+  };
+
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+  const int chunks = static_cast<int>(p.K / 32);
+  const int own = chunks > wave ? (chunks - wave + kSplitWaves - 1) / kSplitWaves : 0;
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    if (s < own) issue(s, wave + s * kSplitWaves);
+  const int r = lane & 31, h = lane >> 5;
+  const int sa = dma_swz<64>(r & 15), sw = sizeof(W) == 4 ? sa : dma_swz<32>(r & 15);
+  int stage = 0;
+  for (int i = 0; i < own; ++i) {
+    // Chunk i has landed once at most the later chunks' DMAs are outstanding.
+    if (i + NS <= own) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * F::kLoads) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const unsigned char* sta = mine + stage * F::kStage + r * 128;
+    const unsigned char* stw = mine + stage * F::kStage + 4096 + r * F::kWRow;
+    if constexpr (sizeof(W) == 4) {
+      u16x8 a[4], w[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        a[g] = *reinterpret_cast<const u16x8*>(sta + 16 * ((2 * g + h) ^ sa));
+        w[g] = *reinterpret_cast<const u16x8*>(stw + 16 * ((2 * g + h) ^ sw));
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) acc = mfma32<W>(w[g], a[g], acc);
+    } else {
+      f32x4 x[2][2];
+      u16x8 w[2];
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          x[g][e] = *reinterpret_cast<const f32x4*>(sta + 16 * ((4 * g + 2 * h + e) ^ sa));
+        w[g] = *reinterpret_cast<const u16x8*>(stw + 16 * ((2 * g + h) ^ sw));
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        uint32_t a[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = x[g][e >> 1][2 * (e & 1)], hi = x[g][e >> 1][2 * (e & 1) + 1];
+          if constexpr (__is_same(W, bf16)) a[e] = pack_bf16x2(lo, hi);
+          else a[e] = pack2(to_bits<W>(lo), to_bits<W>(hi));
+        }
+        acc = mfma32<W>(w[g], __builtin_bit_cast(u16x8, make_uint4(a[0], a[1], a[2], a[3])), acc);
+      }
+    }
+    if (i + NS < own) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read
+      issue(stage, wave + (i + NS) * kSplitWaves);
+    }
+    stage = stage + 1 == NS ? 0 : stage + 1;
+  }
+  __syncthreads();  // every wave is done with its stages
+  f32x4* part = reinterpret_cast<f32x4*>(smem);  // [wave][quad][lane]
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    part[(wave * 4 + q) * kWave + lane] =
+        f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  __syncthreads();
+  // Quad q of lane l holds columns 8q + 4 (l / 32) .. +3 of row l % 32.
+  // Thread -> (row m, column quad nq), columns fastest: a row's pieces leave
+  // side by side.
+  if (tid >= 256) return;
+  const int m = tid >> 3, nq = tid & 7;
+  const int at = (nq >> 1) * kWave + m + 32 * (nq & 1);
+  f32x4 sum = part[at];
+#pragma unroll
+  for (int w = 1; w < kSplitWaves; ++w) sum += part[w * 4 * kWave + at];
+  const int64_t mm = m0 + m, n = n0 + 4 * nq;
+  if (mm >= p.M) return;
+  TO* out = static_cast<TO*>(p.out) + mm * p.ldo + n;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] = sum[e] + (p.bias != nullptr && n + e < p.N ? load_any_f(p.bias, p.bias_dtype, n + e) : 0.0f);
+  if (n + 4 <= p.N && (reinterpret_cast<uintptr_t>(out) & (4 * sizeof(TO) - 1)) == 0) {
+    put4<TO>(out, v[0], v[1], v[2], v[3]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < p.N) out[e] = from_f32<TO>(v[e]);
+  }
+}
+
+template <typename W, typename TO>
+hipError_t launch_split(const GemmParams& p, hipStream_t s) {
+  constexpr size_t lds = SplitForm<W>::kLds;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&split_kernel<W, TO>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+  if (attr != hipSuccess) {
+    set_error("linear: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr));
+    return attr;
+  }
+  const int64_t tiles = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+  hipLaunchKernelGGL((split_kernel<W, TO>), dim3(static_cast<unsigned>(tiles)),
+                     dim3(kSplitWaves * kWave), lds, s, p);
+  return launch_status("linear");
+}
+
+// ---------------------------------------------------------------------------
+// 16-bit A and W, K = 32 KS <= 128: W in registers, A tiles streamed
+// ---------------------------------------------------------------------------
+//
+// The expanded-cache projection writes 2H columns from a K of 32..128: its
+// output is 10-50 times its input, so the stores bound it.  A workgroup of four
+// waves owns 128 output columns: each wave keeps the W fragments of its 32
+// columns in registers for the whole kernel and the workgroup walks 64-row
+// tiles of A.  Tile i + 1 comes into LDS by LDS-DMA while tile i is multiplied,
+// and the tile's outputs are restaged in LDS and leave as whole 256-byte row
+// segments (128 16-bit columns).  ~50 KB of LDS, so three workgroups share a CU
+// and one's stores overlap another's loads and products.  The sums take the
+// same k-steps as smallk_kernel's (bits equal).
+template <typename TO, int KS>
+constexpr size_t stream_lds_bytes() {
+  return 2 * 64 * 32 * KS * 2 + 64 * (128 * sizeof(TO) + 16);
+}
+
+template <typename W, typename TO, int KS>
+__global__ void __launch_bounds__(256) smallk_stream_kernel(const GemmParams p, int row_tiles) {
+  constexpr int K = 32 * KS;
+  constexpr int QPR = K / 8;                       // 16-byte pieces per row
+  constexpr int SW = QPR % 16 == 0 ? 16 : (QPR % 8 == 0 ? 8 : 4);
+  constexpr int kTile = 64 * K * 2;                // bytes of an A tile
+  constexpr int kDma = kTile / 16 / 256;           // DMA instructions per wave and tile
+  constexpr int kOut = 128 * static_cast<int>(sizeof(TO)) + 16;  // staged row stride (bytes)
+  constexpr int kPieces = 64 * 128 * static_cast<int>(sizeof(TO)) / 16 / 256;  // per thread
+  constexpr int kRowPieces = 128 * static_cast<int>(sizeof(TO)) / 16;
+  extern __shared__ __align__(16) unsigned char smem[];
+  unsigned char* stage = smem + 2 * kTile;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r16 = lane & 15, g = lane >> 4;
+  // Workgroup -> (row group, column tile): column tiles of one row group are
+  // consecutive logical workgroups, on one XCD, so A is read into one L2.
+  const int64_t tiles_n = p.N / 128;
+  const int64_t wg = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t nt = (wg % tiles_n) * 128;
+  const int64_t t0 = (wg / tiles_n) * row_tiles;
+  const int64_t all = (p.M + 63) / 64;
+  const int nrt = static_cast<int>(all - t0 < row_tiles ? all - t0 : row_tiles);
+  const rsrc_t ar = make_rsrc(p.a, p.a_bytes);
+  const uint32_t lda_b = static_cast<uint32_t>(p.lda * 2);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
+
+  // LDS piece q of tile row r holds the row's piece q ^ (r % SW).
+  uint32_t src[kDma];
+  int srow[kDma];
+#pragma unroll
+  for (int d = 0; d < kDma; ++d) {
+    const int piece = (wave * kDma + d) * kWave + lane;
+    srow[d] = piece / QPR;
+    src[d] = static_cast<uint32_t>((piece % QPR) ^ (srow[d] % SW)) * 16u;
+  }
+  auto issue = [&](int i) {
+    const int64_t m = (t0 + i) * 64;
+#pragma unroll
+    for (int d = 0; d < kDma; ++d) {
+      const uint32_t off = m + srow[d] < p.M
+                               ? static_cast<uint32_t>(m + srow[d]) * lda_b + src[d]
+                               : kNoOffset;
+      lds_dma16(ar, lds0 + (i & 1) * kTile + (wave * kDma + d) * 1024u, off);
+    }
+  };
+  issue(0);
+  // The wave's W fragments (columns nt + 32 wave + 16 j + r16) and its lanes'
+  // output bias (columns nt + 32 wave + 16 j + 4 g + e).
+  const int n0 = 32 * wave;
+  u16x8 b[KS][2];
+  const W* wt = static_cast<const W*>(p.w);
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      b[s][j] = *reinterpret_cast<const u16x8*>(wt + (nt + n0 + 16 * j + r16) * K + 32 * s + 8 * g);
+  float bv[2][4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      bv[j][e] = p.bias != nullptr ? load_any_f(p.bias, p.bias_dtype, nt + n0 + 16 * j + 4 * g + e) : 0.0f;
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+
+  for (int i = 0; i < nrt; ++i) {
+    // Tile i has landed: its DMAs were followed by the stores of tile i - 1 only.
+    if (i > 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(kPieces));
+    __syncthreads();  // tile i in LDS, tile i - 1 and the staged rows read by every wave
+    if (i + 1 < nrt) issue(i + 1);
+    const unsigned char* tile = smem + (i & 1) * kTile;
+    f32x4 acc[4][2];
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[x][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int q = 4 * s + g;
+      u16x8 a[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        a[x] = *reinterpret_cast<const u16x8*>(tile + (16 * x + r16) * (2 * K) + 16 * (q ^ (r16 % SW)));
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[x][j] = mfma16<W>(b[s][j], a[x], acc[x][j]);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        put4<TO>(reinterpret_cast<TO*>(stage + (16 * x + r16) * kOut) + n0 + 16 * j + 4 * g,
+                 acc[x][j][0] + bv[j][0], acc[x][j][1] + bv[j][1], acc[x][j][2] + bv[j][2],
+                 acc[x][j][3] + bv[j][3]);
+    __syncthreads();  // the tile's outputs staged
+    const int64_t m = (t0 + i) * 64;
+    TO* out = static_cast<TO*>(p.out);
+#pragma unroll
+    for (int t = 0; t < kPieces; ++t) {
+      const int piece = t * 256 + tid;
+      const int r = piece / kRowPieces, c = piece % kRowPieces;
+      const uint4 v = *reinterpret_cast<const uint4*>(stage + r * kOut + 16 * c);
+      if (m + r < p.M)
+        *reinterpret_cast<uint4*>(reinterpret_cast<unsigned char*>(out + (m + r) * p.ldo + nt) + 16 * c) = v;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
 
@@ -992,6 +1319,69 @@ hipError_t launch_dma(const GemmParams& p, hipStream_t s) {
   }
   const int64_t tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(WM * WN * kWave), lds, s, p);
+  return launch_status("linear");
+}
+
+template <typename W, typename TO, int KS>
+hipError_t launch_stream(const GemmParams& p, hipStream_t s) {
+  constexpr size_t lds = stream_lds_bytes<TO, KS>();
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&smallk_stream_kernel<W, TO, KS>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+  if (attr != hipSuccess) {
+    set_error("linear: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr));
+    return attr;
+  }
+  // Row tiles per workgroup: three workgroups per CU when there is enough work,
+  // one tile each otherwise.
+  const int64_t rows = (p.M + 63) / 64, cols = p.N / 128;
+  const int64_t per = (rows * cols + 767) / 768;
+  const int64_t groups = (rows + per - 1) / per;
+  hipLaunchKernelGGL((smallk_stream_kernel<W, TO, KS>), dim3(static_cast<unsigned>(groups * cols)),
+                     dim3(256), lds, s, p, static_cast<int>(per));
+  return launch_status("linear");
+}
+
+// Whether split_kernel takes this problem: whole 32-wide chunks of K, 16-byte
+// aligned rows and operands within its 32-bit offsets.
+inline bool split_fits(const GemmParams& p) {
+  return p.K % 32 == 0 && p.lda % 4 == 0 && p.a_bytes != 0 &&
+         (reinterpret_cast<uintptr_t>(p.a) & 15u) == 0 &&
+         (reinterpret_cast<uintptr_t>(p.w) & 15u) == 0;
+}
+
+// fp32 weights.
+template <typename TO>
+hipError_t launch_f32(const GemmParams& p, hipStream_t s) {
+  // split / skinny / 64x64 DMA tiles / f32_tile, us:
+  //   M=1 N=512 K=576       5.6 / 4.6 / 12.7 / 42     M=4 N=4608 K=128  3.6 / 7.1 / 4.8 / 11.9
+  //   M=64 N=576 K=2304    12.0 / 14.8 / 44 / 198     M=128 N=2048 K=128  3.9 / - / 5.3 / 15
+  //   M=1024 N=256 K=1024   7.9 / - / 21.6 / 89       M=1024 N=512 K=512 (512 split tiles)  10.1 / - / 12.6 / 47
+  //   M=1024 N=2048 K=128  21.3 / - / 9.1 / 23        M=15360 N=512 K=512  126 / - / 79 / 231
+  const int64_t t32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+  const bool aligned = p.lda % 4 == 0 && (reinterpret_cast<uintptr_t>(p.a) & 15u) == 0 &&
+                       (reinterpret_cast<uintptr_t>(p.w) & 15u) == 0;
+  const bool split = split_fits(p) && (t32 <= 256 || (t32 <= 512 && p.K >= 512));
+  if (p.M <= kSkinnyM && p.a_bytes != 0 && p.K % 4 == 0 && aligned &&
+      !(split && (p.M > 32 || p.K < 256))) {
+    const dim3 grid(static_cast<unsigned>((p.N + 4 * kF32SkinnyCols - 1) / (4 * kF32SkinnyCols)),
+                    static_cast<unsigned>((p.M + kF32SkinnyRows - 1) / kF32SkinnyRows));
+    hipLaunchKernelGGL((f32_skinny_kernel<TO>), grid, dim3(256), 0, s, p);
+    return launch_status("linear");
+  }
+  if (split) return launch_split<float, TO>(p, s);
+  constexpr int64_t kLimit = int64_t(1) << 31;
+  if (aligned && p.K % 32 == 0 && (p.ldo * static_cast<int64_t>(sizeof(TO))) % 16 == 0 &&
+      (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0 && 64 * p.lda * 4 < kLimit &&
+      64 * p.K * 4 < kLimit) {
+    // The DMA tile kernel counts K and row strides in 16-bit units.
+    GemmParams q = p;
+    q.K = 2 * p.K;
+    q.lda = 2 * p.lda;
+    return launch_dma<float, TO, 64, 64, 2, 2, 2, kDmaSliceK>(q, s);
+  }
+  const dim3 grid(static_cast<unsigned>(((p.M + 63) / 64) * ((p.N + 63) / 64)));
+  hipLaunchKernelGGL((f32_tile_kernel<TO>), grid, dim3(256), 0, s, p);
   return launch_status("linear");
 }
 
@@ -1024,6 +1414,18 @@ hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
     return launch_status("linear");
   }
   const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128);
+  if constexpr (__is_same(TA, W)) {
+    if (p.K <= 128 && p.K % 32 == 0 && p.a_bytes != 0 && p.N % 128 == 0 &&
+        (p.ldo * static_cast<int64_t>(sizeof(TO))) % 16 == 0 &&
+        (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0) {
+      switch (p.K / 32) {
+        case 1: return launch_stream<W, TO, 1>(p, s);
+        case 2: return launch_stream<W, TO, 2>(p, s);
+        case 3: return launch_stream<W, TO, 3>(p, s);
+        default: return launch_stream<W, TO, 4>(p, s);
+      }
+    }
+  }
   if (p.K <= 128 && p.K % 32 == 0 && p.a_bytes != 0) {
     const dim3 grid(static_cast<unsigned>(big));
     switch (p.K / 32) {
@@ -1081,10 +1483,22 @@ hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
   }
   if (dma_fits<TA, W, TO>(p)) {
     // 256x256 tiles (eight waves of 128x64) once they fill the chip; 128x128
-    // (four waves, two workgroups per CU) below that.
+    // (four waves, two workgroups per CU) below that; 64x64 where even those are
+    // fewer than the CUs.  The k order is the same, so are the bits.  128 vs 64:
+    // M=3584 N=512 K=576 (112 tiles) 8.7 / 6.9 us, M=4096 N=768 K=3072 (192)
+    // 35.7 / 31.7, M=8192 N=512 K=576 (256) 10.6 / 12.1.
     if (((p.M + 255) / 256) * ((p.N + 255) / 256) >= 256)
       return launch_dma<W, TO, 256, 256, 2, 4, 2, kDmaSliceK>(p, s);
-    return launch_dma<W, TO, 128, 128, 2, 2, 2, kDmaSliceK>(p, s);
+    if (big >= 256) return launch_dma<W, TO, 128, 128, 2, 2, 2, kDmaSliceK>(p, s);
+    return launch_dma<W, TO, 64, 64, 2, 2, 2, kDmaSliceK>(p, s);
+  }
+  if constexpr (sizeof(TA) == 4) {
+    // Few tiles: a 64x128 tile's K loop is a chain the chip waits on.  split /
+    // tile64, us: M=192 N=576 K=2304 6.6 / 41.4, M=1024 N=512 K=1024 9.5 / 21.5,
+    // M=2048 N=512 K=512 (1024 split tiles) 12.7 / 14.2; M=4096 N=512 K=1024
+    // (2048) 31.6 / 23.3.
+    const int64_t t32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+    if (split_fits(p) && t32 <= (p.K >= 512 ? 1024 : 512)) return launch_split<W, TO>(p, s);
   }
   if (big >= 256) {
     hipLaunchKernelGGL((tile_kernel<TA, W, TO, 128, 128>), dim3(static_cast<unsigned>(big)),
@@ -1163,27 +1577,9 @@ hipError_t linear_impl(const rlm_tensor* input, const rlm_tensor* weight, const 
   if (weight->dtype == RLM_F32) {
     RLM_REQUIRE(input->dtype == RLM_F32, "%s: fp32 weights need fp32 input (got %s)", what,
                 dtype_name(input->dtype));
-    if (M <= kSkinnyM && p.a_bytes != 0 && K % 4 == 0 && p.lda % 4 == 0 &&
-        (reinterpret_cast<uintptr_t>(input->data) & 15u) == 0 &&
-        (reinterpret_cast<uintptr_t>(weight->data) & 15u) == 0) {
-      const dim3 grid(static_cast<unsigned>((N + 4 * kF32SkinnyCols - 1) / (4 * kF32SkinnyCols)),
-                      static_cast<unsigned>((M + kF32SkinnyRows - 1) / kF32SkinnyRows));
-      if (out->dtype == RLM_F32)
-        hipLaunchKernelGGL((f32_skinny_kernel<float>), grid, dim3(256), 0, stream, p);
-      else if (out->dtype == RLM_BF16)
-        hipLaunchKernelGGL((f32_skinny_kernel<bf16>), grid, dim3(256), 0, stream, p);
-      else
-        hipLaunchKernelGGL((f32_skinny_kernel<f16>), grid, dim3(256), 0, stream, p);
-      return launch_status(what);
-    }
-    const dim3 grid(static_cast<unsigned>(((M + 63) / 64) * ((N + 63) / 64)));
-    if (out->dtype == RLM_F32)
-      hipLaunchKernelGGL((f32_tile_kernel<float>), grid, dim3(256), 0, stream, p);
-    else if (out->dtype == RLM_BF16)
-      hipLaunchKernelGGL((f32_tile_kernel<bf16>), grid, dim3(256), 0, stream, p);
-    else
-      hipLaunchKernelGGL((f32_tile_kernel<f16>), grid, dim3(256), 0, stream, p);
-    return launch_status(what);
+    if (out->dtype == RLM_F32) return launch_f32<float>(p, stream);
+    if (out->dtype == RLM_BF16) return launch_f32<bf16>(p, stream);
+    return launch_f32<f16>(p, stream);
   }
   RLM_REQUIRE(K % 8 == 0 && p.lda % 8 == 0,
               "%s: reduction dim and input row stride must be multiples of 8 for 16-bit weights",
