@@ -24,6 +24,8 @@
 
 #include "rlm_common.hpp"
 
+#include <type_traits>
+
 namespace rlm {
 namespace {
 
@@ -890,7 +892,13 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
     wave_sync();  // the staging is read before it is written again
   };
 
-  // Prologue: chunk 0's hidden, then the first W2 k-groups of chunk 0.
+  // Prologue: chunk 0's hidden, then the first W2 k-groups of chunk 0.  Loads
+  // past the last chunk repeat the last one: every load of the loop is issued
+  // unconditionally, so the compiler's waits count exactly the loads between an
+  // operand's and its use.  (With `if (c + 2 < nchunks)` around the W_m and
+  // cache loads it had to assume them absent and waited, each chunk, for loads
+  // that were only needed a chunk later.)
+  const int last = nchunks - 1;
   u16x8 wq[K2][TNB];
   {
     f32x16 hacc;
@@ -898,25 +906,18 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
     for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) p1_step(hacc, kk);
-    if (nchunks > 1) load_wm(1);
+    load_wm(min(1, last));
 #pragma unroll
     for (int s = 0; s < kMlpW2Ahead; ++s) load_w2(wq[s], s);
     p1_epilogue(hacc, hid);
-    if (nchunks > 1) load_x(1);
+    load_x(min(1, last));
   }
   __syncthreads();  // hidden chunk 0 complete
 
-  // Iteration c: phase 2 of chunk c with phase 1's matrix work for chunk c + 1
+  // Phase 2 of chunk c; P1: with phase 1's matrix work for chunk c + 1
   // interleaved (one k-step per k-group: independent of phase 2, it fills the
-  // matrix pipeline around phase 2's products), then chunk c + 1's epilogue into
-  // the other hidden buffer.  The last iteration's phase-1 products are
-  // discarded (no branch in the k-loop).
-  for (int c = 0; c < nchunks; ++c) {
-    unsigned char* hb = hid + (c & 1) * (kMlpRows * kMlpHidRow);
-    unsigned char* hn = hid + ((c + 1) & 1) * (kMlpRows * kMlpHidRow);
-    f32x16 hacc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
+  // matrix pipeline around phase 2's products).
+  auto phase2 = [&](int c, const unsigned char* hb, f32x16& hacc, auto p1) {
 #pragma unroll
     for (int s = 0; s < K2; ++s) {
       if (s + kMlpW2Ahead < K2) load_w2(wq[s + kMlpW2Ahead], c * K2 + s + kMlpW2Ahead);
@@ -930,16 +931,28 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
         for (int i = 0; i < 2; ++i)
           acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               __builtin_bit_cast(bf16x8, wq[s][j]), __builtin_bit_cast(bf16x8, fa[i]), acc[j][i], 0, 0, 0);
-      if (s < KK) p1_step(hacc, s);
+      if (decltype(p1)::value && s < KK) p1_step(hacc, s);
     }
-    if (c + 1 < nchunks) {  // uniform
-      if (c + 2 < nchunks) load_wm(c + 2);
+  };
+  // Iteration c: phase 2 of chunk c, then chunk c + 1's epilogue into the other
+  // hidden buffer; the last chunk's phase 2 follows the loop.
+  for (int c = 0; c < last; ++c) {
+    unsigned char* hb = hid + (c & 1) * (kMlpRows * kMlpHidRow);
+    unsigned char* hn = hid + ((c + 1) & 1) * (kMlpRows * kMlpHidRow);
+    f32x16 hacc;
 #pragma unroll
-      for (int s = 0; s < kMlpW2Ahead; ++s) load_w2(wq[s], (c + 1) * K2 + s);
-      p1_epilogue(hacc, hn);
-      if (c + 2 < nchunks) load_x(c + 2);
-    }
+    for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
+    phase2(c, hb, hacc, std::true_type{});
+    load_wm(min(c + 2, last));
+#pragma unroll
+    for (int s = 0; s < kMlpW2Ahead; ++s) load_w2(wq[s], (c + 1) * K2 + s);
+    p1_epilogue(hacc, hn);
+    load_x(min(c + 2, last));
     __syncthreads();  // phase 2 of chunk c read; hidden chunk c + 1 complete
+  }
+  {
+    f32x16 none;
+    phase2(last, hid + (last & 1) * (kMlpRows * kMlpHidRow), none, std::false_type{});
   }
 
   // ---- Output: acc[j][i] holds raw[row 32i + (lane & 31)][columns dw0 + 32j +
