@@ -699,7 +699,6 @@ constexpr int kMlpThreads = kMlpWaves * kWave;
 constexpr int kMlpChunk = 128;                  // hidden columns per chunk
 constexpr int kMlpHidRow = kMlpChunk * 2 + 16;  // LDS hidden row (bytes): conflict-free 16-byte reads
 constexpr int kMlpStageRow = 32 * 4 + 16;       // phase-1 restaged fp32 row (bytes)
-constexpr int kMlpW2Ahead = 2;                  // W2 k-groups loaded ahead of their products
 
 // Both weights arrive in MFMA fragment order (rlm_mfma_fragments): fragment
 // (n-block nb, k-group g) of a [N, K] weight is 64 lanes x 8 consecutive k,
@@ -773,31 +772,26 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   // Phase-1 roles: row block i1 and column block j1 (32 hidden columns of the
   // chunk).  W_m fragment kk: rows c*128 + 32 j1 .. +31, k-group kk.
   const int i1 = wave & 1, j1 = wave >> 1;
-  u16x8 fwm[KK];
-  auto load_wm = [&](int c) {
+  auto load_wm = [&](int c, int kk) {
     const uint32_t nb = static_cast<uint32_t>(c * (kMlpChunk / 32) + j1);
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk)
-      fwm[kk] = __builtin_bit_cast(u16x8, buf_load_b128(wr, ((nb * KK + kk) * kWave + lane) * 16u));
+    return __builtin_bit_cast(u16x8, buf_load_b128(wr, ((nb * KK + kk) * kWave + lane) * 16u));
   };
   // Row-contiguous roles of the phase-1 epilogue: piece t is row 16t + (lane >> 2)
   // of the block, columns 8 (lane & 3) .. +7 of its 32.  Rows outside the
   // caches have kNoOffset bases: their gathers read zeros.
   const int c8 = 8 * (lane & 3);
   uint4 xa[2], xp[2];
-  auto load_x = [&](int c) {
+  auto load_x = [&](int c, int t) {
     const uint32_t n = static_cast<uint32_t>(c * kMlpChunk + 32 * j1 + c8);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int m = 32 * i1 + 16 * t + (lane >> 2);
-      xa[t] = buf_load_b128(xr, rt.x_a[m] + 2u * n);
-      xp[t] = buf_load_b128(xr, rt.x_p[m] + 2u * n);
-    }
+    const int m = 32 * i1 + 16 * t + (lane >> 2);
+    xa[t] = buf_load_b128(xr, rt.x_a[m] + 2u * n);
+    xp[t] = buf_load_b128(xr, rt.x_p[m] + 2u * n);
   };
 
   // Set-up: row table, then the products (every load of a thread issued first).
   load_rows<bf16, kMlpRows>(p, r0, rt);
   __syncthreads();
+  u16x8 fwm[KK];  // chunk 0's W_m fragments (the loop streams the later chunks')
   {
     uint4 va[kPieces], vp[kPieces];
 #pragma unroll
@@ -807,8 +801,10 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
       va[c] = buf_load_b128(opr, rt.op_a[row] + 16u * q);
       vp[c] = buf_load_b128(opr, rt.op_p[row] + 16u * q);
     }
-    load_wm(0);
-    load_x(0);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) fwm[kk] = load_wm(0, kk);
+    load_x(0, 0);
+    load_x(0, 1);
 #pragma unroll
     for (int c = 0; c < kPieces; ++c) {
       const int piece = c * kMlpThreads + tid;
@@ -836,12 +832,24 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   // k-group g: n-block TNB w + j, k-group g.
   const int dw0 = 32 * TNB * wave;
   const uint32_t kgroups = H / 16u;
-  auto load_w2 = [&](u16x8 (&w)[TNB], int g) {
+  const int last = nchunks - 1;
+  // The weight stream.  Step s of chunk c takes W2's k-group (c, s) and, for phase
+  // 1 of chunk c + 1, W_m's k-group s: one slot of a ring of four, loaded three
+  // steps (one slot) ahead and straight through the chunk ends.  Every load is
+  // unconditional (past the last chunk it repeats the last one), so that the
+  // compiler's waits count exactly the loads between an operand's and its use.
+  constexpr int kRing = 4;
+  static_assert(K2 % kRing == 0 && K2 >= KK, "the ring's slots are static");
+  u16x8 w2q[kRing][TNB], wmq[kRing];
+  auto load_step = [&](int c, int s) {
+    const int slot = s % kRing;
+    const int g = min(c, last) * K2 + s;
 #pragma unroll
     for (int j = 0; j < TNB; ++j)
-      w[j] = __builtin_bit_cast(
+      w2q[slot][j] = __builtin_bit_cast(
           u16x8, buf_load_b128(w2r, ((static_cast<uint32_t>(TNB * wave + j) * kgroups + g) * kWave +
                                      lane) * 16u));
+    if (s < KK) wmq[slot] = load_wm(min(c + 1, last), s);
   };
   // Hidden-tile A fragments: row 32i + (lane & 31), k = 16s + 8 (lane >> 5) of the chunk.
   const int hid_lane = (lane & 31) * kMlpHidRow + 16 * (lane >> 5);
@@ -856,18 +864,17 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
 
   // Phase 1 of a chunk, one k-step: hidden^T block (columns 32 j1.., rows
   // 32 i1..) += W_m fragment kk . product fragments (hi, then lo).
-  auto p1_step = [&](f32x16& hacc, int kk) {
-    const int off = prod_off + (((2 * kk + (lane >> 5)) ^ swz) << 4);
-    const u16x8 fh = *reinterpret_cast<const u16x8*>(p_hi + off);
-    const u16x8 fl = *reinterpret_cast<const u16x8*>(p_lo + off);
-    hacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fwm[kk]),
-                                                   __builtin_bit_cast(bf16x8, fh), hacc, 0, 0, 0);
-    hacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fwm[kk]),
-                                                   __builtin_bit_cast(bf16x8, fl), hacc, 0, 0, 0);
+  auto product = [&](const unsigned char* part, int kk) {
+    return *reinterpret_cast<const u16x8*>(part + prod_off + (((2 * kk + (lane >> 5)) ^ swz) << 4));
+  };
+  auto p1_mfma = [&](f32x16& hacc, const u16x8& w, const u16x8& f) {
+    hacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w),
+                                                   __builtin_bit_cast(bf16x8, f), hacc, 0, 0, 0);
   };
   // Its epilogue: + expanded-cache halves (xa / xp), GELU, bf16 into hidden
-  // buffer hb.  hacc: lane holds hidden^T[column 8q + 4 (lane >> 5) + e][row lane & 31].
-  auto p1_epilogue = [&](const f32x16& hacc, unsigned char* hb) {
+  // buffer hb; each half's registers take chunk cx's as soon as they are read.
+  // hacc: lane holds hidden^T[column 8q + 4 (lane >> 5) + e][row lane & 31].
+  auto p1_epilogue = [&](const f32x16& hacc, unsigned char* hb, int cx) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       *reinterpret_cast<float4*>(stage + (lane & 31) * kMlpStageRow + (8 * q + 4 * (lane >> 5)) * 4) =
@@ -884,54 +891,67 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
       float v[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[2 * e] = gelu_erf(sv[2 * e] + (bf16_lo(a[e]) + bf16_lo(b[e])));
-        v[2 * e + 1] = gelu_erf(sv[2 * e + 1] + (bf16_hi(a[e]) + bf16_hi(b[e])));
+        v[2 * e] = sv[2 * e] + (bf16_lo(a[e]) + bf16_lo(b[e]));
+        v[2 * e + 1] = sv[2 * e + 1] + (bf16_hi(a[e]) + bf16_hi(b[e]));
       }
+      load_x(cx, t);
+      __builtin_amdgcn_sched_barrier(0);  // the loads go out before the GELUs
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
       put8<bf16>(reinterpret_cast<bf16*>(hb + (32 * i1 + row) * kMlpHidRow + (32 * j1 + c8) * 2), v);
     }
     wave_sync();  // the staging is read before it is written again
   };
 
-  // Prologue: chunk 0's hidden, then the first W2 k-groups of chunk 0.  Loads
-  // past the last chunk repeat the last one: every load of the loop is issued
-  // unconditionally, so the compiler's waits count exactly the loads between an
-  // operand's and its use.  (With `if (c + 2 < nchunks)` around the W_m and
-  // cache loads it had to assume them absent and waited, each chunk, for loads
-  // that were only needed a chunk later.)
-  const int last = nchunks - 1;
-  u16x8 wq[K2][TNB];
+  // Prologue: chunk 0's hidden and the first steps of the weight stream.
   {
     f32x16 hacc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) p1_step(hacc, kk);
-    load_wm(min(1, last));
+    for (int kk = 0; kk < KK; ++kk) {
+      p1_mfma(hacc, fwm[kk], product(p_hi, kk));
+      p1_mfma(hacc, fwm[kk], product(p_lo, kk));
+    }
 #pragma unroll
-    for (int s = 0; s < kMlpW2Ahead; ++s) load_w2(wq[s], s);
-    p1_epilogue(hacc, hid);
-    load_x(min(1, last));
+    for (int s = 0; s < kRing - 1; ++s) load_step(0, s);
+    p1_epilogue(hacc, hid, min(1, last));
   }
   __syncthreads();  // hidden chunk 0 complete
 
-  // Phase 2 of chunk c; P1: with phase 1's matrix work for chunk c + 1
-  // interleaved (one k-step per k-group: independent of phase 2, it fills the
-  // matrix pipeline around phase 2's products).
+  // Phase 2 of chunk c; P1: with phase 1's matrix work for chunk c + 1 (one
+  // k-step per step).  LDS fragments are read a step ahead; the scheduling
+  // barriers keep loads, reads and products of a step together -- left alone,
+  // the compiler sinks the weight loads to their uses.
   auto phase2 = [&](int c, const unsigned char* hb, f32x16& hacc, auto p1) {
-#pragma unroll
-    for (int s = 0; s < K2; ++s) {
-      if (s + kMlpW2Ahead < K2) load_w2(wq[s + kMlpW2Ahead], c * K2 + s + kMlpW2Ahead);
-      u16x8 fa[2];
+    constexpr bool kP1 = decltype(p1)::value;
+    u16x8 fa[2][2], fh[2], fl[2];
+    auto read = [&](int s) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        fa[i] = *reinterpret_cast<const u16x8*>(hb + 32 * i * kMlpHidRow + hid_lane + 32 * s);
+        fa[s & 1][i] = *reinterpret_cast<const u16x8*>(hb + 32 * i * kMlpHidRow + hid_lane + 32 * s);
+      if (kP1 && s < KK) {
+        fh[s & 1] = product(p_hi, s);
+        fl[s & 1] = product(p_lo, s);
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int s = 0; s < K2; ++s) {
+      if (kP1 || s + kRing - 1 < K2)
+        load_step(c + (s + kRing - 1) / K2, (s + kRing - 1) % K2);
+      if (s + 1 < K2) read(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kP1 && s < KK) p1_mfma(hacc, wmq[s % kRing], fh[s & 1]);
 #pragma unroll
       for (int j = 0; j < TNB; ++j)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
           acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              __builtin_bit_cast(bf16x8, wq[s][j]), __builtin_bit_cast(bf16x8, fa[i]), acc[j][i], 0, 0, 0);
-      if (decltype(p1)::value && s < KK) p1_step(hacc, s);
+              __builtin_bit_cast(bf16x8, w2q[s % kRing][j]), __builtin_bit_cast(bf16x8, fa[s & 1][i]),
+              acc[j][i], 0, 0, 0);
+      if (kP1 && s < KK) p1_mfma(hacc, wmq[s % kRing], fl[s & 1]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   // Iteration c: phase 2 of chunk c, then chunk c + 1's epilogue into the other
@@ -943,11 +963,7 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
 #pragma unroll
     for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
     phase2(c, hb, hacc, std::true_type{});
-    load_wm(min(c + 2, last));
-#pragma unroll
-    for (int s = 0; s < kMlpW2Ahead; ++s) load_w2(wq[s], (c + 1) * K2 + s);
-    p1_epilogue(hacc, hn);
-    load_x(min(c + 2, last));
+    p1_epilogue(hacc, hn, min(c + 2, last));
     __syncthreads();  // phase 2 of chunk c read; hidden chunk c + 1 complete
   }
   {
