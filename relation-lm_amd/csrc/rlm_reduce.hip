@@ -834,10 +834,11 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   const uint32_t kgroups = H / 16u;
   const int last = nchunks - 1;
   // The weight stream.  Step s of chunk c takes W2's k-group (c, s) and, for phase
-  // 1 of chunk c + 1, W_m's k-group s: one slot of a ring of four, loaded three
+  // 1 of chunk c + 1 (late waves, see below: c + 2), W_m's k-group s: one slot of a ring of four, loaded three
   // steps (one slot) ahead and straight through the chunk ends.  Every load is
   // unconditional (past the last chunk it repeats the last one), so that the
   // compiler's waits count exactly the loads between an operand's and its use.
+  const int late = wave >> 2;
   constexpr int kRing = 4;
   static_assert(K2 % kRing == 0 && K2 >= KK, "the ring's slots are static");
   u16x8 w2q[kRing][TNB], wmq[kRing];
@@ -849,7 +850,7 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
       w2q[slot][j] = __builtin_bit_cast(
           u16x8, buf_load_b128(w2r, ((static_cast<uint32_t>(TNB * wave + j) * kgroups + g) * kWave +
                                      lane) * 16u));
-    if (s < KK) wmq[slot] = load_wm(min(c + 1, last), s);
+    if (s < KK) wmq[slot] = load_wm(min(c + 1 + late, last), s);
   };
   // Hidden-tile A fragments: row 32i + (lane & 31), k = 16s + 8 (lane >> 5) of the chunk.
   const int hid_lane = (lane & 31) * kMlpHidRow + 16 * (lane >> 5);
@@ -903,24 +904,34 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
     wave_sync();  // the staging is read before it is written again
   };
 
-  // Prologue: chunk 0's hidden and the first steps of the weight stream.
-  {
-    f32x16 hacc;
+  // Prologue: chunk 0's hidden (late waves: and chunk 1's sums) and the first
+  // steps of the weight stream.
+  f32x16 hacc;
+  auto p1_zero = [&]() {
 #pragma unroll
     for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
+  };
+  auto p1_whole = [&]() {
+    p1_zero();
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       p1_mfma(hacc, fwm[kk], product(p_hi, kk));
       p1_mfma(hacc, fwm[kk], product(p_lo, kk));
     }
+  };
+  p1_whole();
+  p1_epilogue(hacc, hid, min(1, last));
+  if (late) {
 #pragma unroll
-    for (int s = 0; s < kRing - 1; ++s) load_step(0, s);
-    p1_epilogue(hacc, hid, min(1, last));
+    for (int kk = 0; kk < KK; ++kk) fwm[kk] = load_wm(min(1, last), kk);
+    p1_whole();
   }
+#pragma unroll
+  for (int s = 0; s < kRing - 1; ++s) load_step(0, s);
   __syncthreads();  // hidden chunk 0 complete
 
-  // Phase 2 of chunk c; P1: with phase 1's matrix work for chunk c + 1 (one
-  // k-step per step).  LDS fragments are read a step ahead; the scheduling
+  // Phase 2 of chunk c; P1: with phase 1's matrix work for chunk c + 1 (late
+  // waves: c + 2), one k-step per step.  LDS fragments are read a step ahead; the scheduling
   // barriers keep loads, reads and products of a step together -- left alone,
   // the compiler sinks the weight loads to their uses.
   auto phase2 = [&](int c, const unsigned char* hb, f32x16& hacc, auto p1) {
@@ -954,16 +965,17 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // Iteration c: phase 2 of chunk c, then chunk c + 1's epilogue into the other
-  // hidden buffer; the last chunk's phase 2 follows the loop.
+  // Iteration c: phase 2 of chunk c and chunk c + 1's epilogue into the other
+  // hidden buffer.  Two waves share a SIMD (w and w + 4): the early four run the
+  // epilogue after their products, the late four before, its sums carried from
+  // the iteration before, so that one wave's GELUs fall on the other's products.
+  // The last chunk's phase 2 follows the loop.
+  auto buffer = [&](int c) { return hid + (c & 1) * (kMlpRows * kMlpHidRow); };
   for (int c = 0; c < last; ++c) {
-    unsigned char* hb = hid + (c & 1) * (kMlpRows * kMlpHidRow);
-    unsigned char* hn = hid + ((c + 1) & 1) * (kMlpRows * kMlpHidRow);
-    f32x16 hacc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) hacc[e] = 0.0f;
-    phase2(c, hb, hacc, std::true_type{});
-    p1_epilogue(hacc, hn, min(c + 2, last));
+    if (late) p1_epilogue(hacc, buffer(c + 1), min(c + 2, last));
+    p1_zero();
+    phase2(c, buffer(c), hacc, std::true_type{});
+    if (!late) p1_epilogue(hacc, buffer(c + 1), min(c + 2, last));
     __syncthreads();  // phase 2 of chunk c read; hidden chunk c + 1 complete
   }
   {
