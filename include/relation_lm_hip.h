@@ -284,6 +284,36 @@ hipError_t rlm_relation_hidden_linear_seq(
     const rlm_tensor* product_weight, const rlm_tensor* second_weight,
     const rlm_tensor* out, hipStream_t stream);
 
+/*
+ * The relation reduce of the sequence form (hidden -> second Linear -> LayerNorm,
+ * active-K softmax and partner sum: the three calls of
+ * benchmarks/benchmark_relation_reduce.py:55-64) with neither intermediate in
+ * memory, like rlm_relation_reduce_fused_seq: 64-row tiles instead of 128 and any
+ * d_model that is a multiple of 32 up to 768.
+ *   expanded_cache [B,T,2H], operand_cache [B,T,R], product_weight [H,R],
+ *   second_weight [D,H] or in MFMA fragment order [D/32,H/16,64,8] (bf16,
+ *   16-byte aligned); anchor_index [B,Tq], partner_index [B,Tq,K] (int32/int64);
+ *   second_bias, norm_weight, norm_bias [D]; partner_scores f32 [B,Tq,K];
+ *   positions [Tq] or [B,Tq];
+ *   workspace bf16 [H*R + D*H] ([H*R] when second_weight is in fragment order),
+ *   16-byte aligned: takes the row-major weights in fragment order.
+ * Output: out f32 [B,Tq,D].  Shapes: R in {64, 128}, H a multiple of 128, D a
+ * multiple of 32 up to 768, K in 1..16 (..._fits says whether given tensors
+ * qualify).
+ */
+hipError_t rlm_relation_mlp_reduce_seq(
+    const rlm_tensor* expanded_cache, const rlm_tensor* operand_cache,
+    const rlm_tensor* anchor_index, const rlm_tensor* partner_index,
+    const rlm_tensor* product_weight, const rlm_tensor* second_weight,
+    const rlm_tensor* second_bias, const rlm_tensor* partner_scores,
+    const rlm_tensor* norm_weight, const rlm_tensor* norm_bias, const rlm_tensor* positions,
+    double norm_eps, const rlm_tensor* workspace, const rlm_tensor* out, hipStream_t stream);
+int rlm_relation_mlp_reduce_seq_fits(const rlm_tensor* expanded_cache,
+                                     const rlm_tensor* operand_cache,
+                                     const rlm_tensor* partner_index,
+                                     const rlm_tensor* product_weight,
+                                     const rlm_tensor* second_weight);
+
 /* 1 if rlm_relation_hidden_linear_seq takes these tensors (dtypes, shapes,
  * alignment; the weights in fragment order), else 0. */
 int rlm_relation_hidden_linear_seq_fits(const rlm_tensor* expanded_cache,

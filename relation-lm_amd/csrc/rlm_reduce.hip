@@ -25,6 +25,7 @@
 #include "rlm_common.hpp"
 
 #include <type_traits>
+#include <utility>
 
 namespace rlm {
 namespace {
@@ -708,9 +709,41 @@ constexpr int kMlpStageRow = 32 * 4 + 16;       // phase-1 restaged fp32 row (by
 struct MlpParams {
   HiddenParams h;      // rows, caches, indices and W_m (fragment order; h.out unused)
   const void* w2;      // second Linear weight [D, H] in fragment order, bf16
-  float* out;          // [rows, D]
+  float* out;          // [rows, D]; reduce forms: [rows / K, D]
   int D;
   uint32_t w2_bytes;
+  // Reduce forms (kMlpQueries, kMlpSlots): what follows the second Linear.
+  const void* b2;      // [D] second Linear bias
+  const void* gamma;   // [D] LayerNorm
+  const void* beta;
+  int b2_dtype, gamma_dtype, beta_dtype;
+  float eps;
+  const float* scores; // [rows] partner scores
+  const void* pos;
+  int pos_dtype;
+  int64_t pos_sb, pos_sq;
+  int tile_rows;       // rows a workgroup takes: whole groups of K, at most kMlpRows
+  // kMlpSlots: anchor slots per query (a group is a (query, slot) pair).
+  int slots;
+  const void* slot_logits;
+  int slot_dtype;
+};
+
+// What a workgroup does with its raw rows.
+//   kMlpRaw      stores them (relation_hidden_linear_seq)
+//   kMlpQueries  bias, LayerNorm, active-K softmax and weighted sum over the K rows
+//                of each query (relation_norm_reduce's epilogue)
+//   kMlpSlots    the same per (query, slot) with the multi-anchor block's weights
+//                (partner softmax times the slot's mixing weight)
+constexpr int kMlpRaw = 0, kMlpQueries = 1, kMlpSlots = 2;
+constexpr int kMlpMaxK = 16;     // partners of the reduce forms
+constexpr int kMlpMaxD = 768;
+
+// Reduce forms: the rows' weights, the waves' row sums and the D-wide vectors.
+struct MlpReduceLds {
+  float weight[kMlpRows];
+  float red[2][kMlpWaves][kMlpRows];
+  float b2[kMlpMaxD], gamma[kMlpMaxD], beta[kMlpMaxD];
 };
 
 // LDS: the hi / lo product tiles, two hidden tiles, the waves' phase-1
@@ -732,14 +765,76 @@ template <int TNB>
 constexpr int mlp_out_row() {
   return 32 * TNB * 4 + 16;
 }
-template <int R, int TNB>
+template <int R>
+constexpr int mlp_reduce_offset() {
+  return (mlp_table_offset<R>() + static_cast<int>(sizeof(RowTableN<kMlpRows>)) + 15) & ~15;
+}
+template <int R, int TNB, int MODE>
 constexpr size_t mlp_lds_bytes() {
+  if (MODE != kMlpRaw) return mlp_reduce_offset<R>() + sizeof(MlpReduceLds);
   constexpr size_t main_bytes = mlp_table_offset<R>() + sizeof(RowTableN<kMlpRows>);
   constexpr size_t out_bytes = static_cast<size_t>(kMlpWaves) * 32 * mlp_out_row<TNB>();
   return main_bytes > out_bytes ? main_bytes : out_bytes;
 }
 
-template <int R, int TNB>
+// Weight of row `row` = K g + k in its group's sum (reduce forms).
+//   kMlpQueries: partner_weight's (relation_reduce.py:399-411);
+//   kMlpSlots:   the slot mix (softmax of the mix logits over the active slots)
+//                times the partner softmax (multi_relation_blocks.py:164-177).
+template <int MODE>
+__device__ float mlp_row_weight(const MlpParams& mp, int64_t row) {
+  const int K = mp.h.K;
+  const int64_t g = row / K;
+  const int k = static_cast<int>(row - g * K);
+  const int64_t per = mp.h.Tq / (MODE == kMlpSlots ? mp.slots : 1);  // queries per batch row
+  const int64_t q = MODE == kMlpSlots ? g / mp.slots : g;
+  const int64_t b = q / per, tq = q - b * per;
+  const int64_t t = index_at(mp.pos, mp.pos_dtype, b * mp.pos_sb + tq * mp.pos_sq);
+  float s[kMlpMaxK];
+#pragma unroll
+  for (int i = 0; i < kMlpMaxK; ++i) s[i] = mp.scores[g * K + (i < K ? i : 0)];
+  int k_limit = K;
+  if (MODE == kMlpQueries) {
+    const int64_t n = t + 1;
+    k_limit = n > 0 ? 64 - __clzll(static_cast<unsigned long long>(n)) : 0;
+    k_limit = k_limit < 1 ? 1 : (k_limit > K ? K : k_limit);
+  }
+  float m = -INFINITY, own = 0.0f, total = 0.0f, active_total = 0.0f;
+  auto active = [&](int i) {
+    return MODE == kMlpQueries ? i < k_limit && s[i] > -1.0e30f
+                               : i < K && s[i] > -INFINITY && s[i] < INFINITY;
+  };
+#pragma unroll
+  for (int i = 0; i < kMlpMaxK; ++i)
+    if (i < K) m = fmaxf(m, active(i) ? s[i] : -1.0e4f);
+#pragma unroll
+  for (int i = 0; i < kMlpMaxK; ++i) {
+    if (i >= K) continue;
+    const float e = expf((active(i) ? s[i] : -1.0e4f) - m);
+    total += e;
+    active_total += active(i) ? e : 0.0f;
+    if (i == k) own = active(i) ? e : 0.0f;
+  }
+  if (MODE == kMlpQueries) return own / fmaxf(active_total, 1.0e-9f);
+  // (e / total) * active / max(sum of those, 1e-9).
+  const float pw = (own / total) / fmaxf(active_total / total, 1.0e-9f);
+  const int slot = static_cast<int>(g - q * mp.slots);
+  float lm = -INFINITY;
+  for (int j = 0; j < mp.slots; ++j) lm = fmaxf(lm, load_any_f(mp.slot_logits, mp.slot_dtype, j));
+  float lsum = 0.0f, asum = 0.0f, mine = 0.0f;
+  for (int j = 0; j < mp.slots; ++j) {
+    const float v = expf(load_any_f(mp.slot_logits, mp.slot_dtype, j) - lm);
+    lsum += v;
+    if (j <= t) asum += v;
+    if (j == slot) mine = v;
+  }
+  return slot <= t ? (mine / lsum) / fmaxf(asum / lsum, 1.0e-9f) * pw : 0.0f;
+}
+
+// RAGGED: d_model / 32 column blocks that do not divide evenly among the waves;
+// the first waves then own one block more (two waves of a SIMD, w and w + 4,
+// together at most one block more than another pair), absent blocks load nothing.
+template <int R, int TNB, int MODE, bool RAGGED>
 __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpParams mp) {
   const HiddenParams& p = mp.h;
   constexpr int PR = R / 8;                               // 16-byte pieces per product row
@@ -758,9 +853,10 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int64_t row_tiles = (p.rows + kMlpRows - 1) / kMlpRows;
+  const int tile_rows = MODE == kMlpRaw ? kMlpRows : mp.tile_rows;
+  const int64_t row_tiles = (p.rows + tile_rows - 1) / tile_rows;
   // Row tiles of neighbouring queries run on one XCD (one L2 for their gathers).
-  const int64_t r0 = xcd_tile(blockIdx.x, row_tiles) * kMlpRows;
+  const int64_t r0 = xcd_tile(blockIdx.x, row_tiles) * tile_rows;
   const int nchunks = p.H / kMlpChunk;
   const uint32_t H = static_cast<uint32_t>(p.H);
   const rsrc_t xr = make_rsrc(p.expanded, p.expanded_bytes);
@@ -789,7 +885,26 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   };
 
   // Set-up: row table, then the products (every load of a thread issued first).
-  load_rows<bf16, kMlpRows>(p, r0, rt);
+  MlpReduceLds& rd = *reinterpret_cast<MlpReduceLds*>(smem + mlp_reduce_offset<R>());
+  if constexpr (MODE == kMlpRaw) {
+    load_rows<bf16, kMlpRows>(p, r0, rt);
+  } else {
+    // Rows past the tile's whole groups are padding (they gather zeros).
+    HiddenParams tile = p;
+    tile.rows = r0 + tile_rows < p.rows ? r0 + tile_rows : p.rows;
+    load_rows<bf16, kMlpRows>(tile, r0, rt);
+    // The second wave forms the rows' weights, the others fetch the vectors.
+    if (wave == 1) {
+      const int64_t row = r0 + lane;
+      rd.weight[lane] = row < tile.rows ? mlp_row_weight<MODE>(mp, row) : 0.0f;
+    } else if (wave > 1) {
+      for (int d = tid - 2 * kWave; d < mp.D; d += kMlpThreads - 2 * kWave) {
+        rd.b2[d] = load_any_f(mp.b2, mp.b2_dtype, d);
+        rd.gamma[d] = load_any_f(mp.gamma, mp.gamma_dtype, d);
+        rd.beta[d] = load_any_f(mp.beta, mp.beta_dtype, d);
+      }
+    }
+  }
   __syncthreads();
   u16x8 fwm[KK];  // chunk 0's W_m fragments (the loop streams the later chunks')
   {
@@ -828,9 +943,12 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   const int swz = tile_swz<PR>(lane & 15);
   const int prod_off = (32 * i1 + (lane & 31)) * RB;
 
-  // Phase-2 roles: D columns dw0 .. dw0 + 32 TNB - 1.  W2 fragment j of global
-  // k-group g: n-block TNB w + j, k-group g.
-  const int dw0 = 32 * TNB * wave;
+  // Phase-2 roles: nb column blocks of 32 from nb0 on (D columns dw0 ..).  W2
+  // fragment j of global k-group g: n-block nb0 + j, k-group g.
+  const int share = mp.D / 32 / kMlpWaves, more = mp.D / 32 % kMlpWaves;
+  const int nb0 = RAGGED ? wave * share + min(wave, more) : TNB * wave;
+  const int nb = RAGGED ? share + (wave < more ? 1 : 0) : TNB;
+  const int dw0 = 32 * nb0;
   const uint32_t kgroups = H / 16u;
   const int last = nchunks - 1;
   // The weight stream.  Step s of chunk c takes W2's k-group (c, s) and, for phase
@@ -848,8 +966,10 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
 #pragma unroll
     for (int j = 0; j < TNB; ++j)
       w2q[slot][j] = __builtin_bit_cast(
-          u16x8, buf_load_b128(w2r, ((static_cast<uint32_t>(TNB * wave + j) * kgroups + g) * kWave +
-                                     lane) * 16u));
+          u16x8, buf_load_b128(w2r, RAGGED && j >= nb
+                                        ? kNoOffset
+                                        : ((static_cast<uint32_t>(nb0 + j) * kgroups + g) * kWave +
+                                           lane) * 16u));
     if (s < KK) wmq[slot] = load_wm(min(c + 1 + late, last), s);
   };
   // Hidden-tile A fragments: row 32i + (lane & 31), k = 16s + 8 (lane >> 5) of the chunk.
@@ -955,12 +1075,14 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
       __builtin_amdgcn_sched_barrier(0);
       if (kP1 && s < KK) p1_mfma(hacc, wmq[s % kRing], fh[s & 1]);
 #pragma unroll
-      for (int j = 0; j < TNB; ++j)
+      for (int j = 0; j < TNB; ++j) {
+        if (RAGGED && j == TNB - 1 && nb < TNB) break;  // uniform
 #pragma unroll
         for (int i = 0; i < 2; ++i)
           acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               __builtin_bit_cast(bf16x8, w2q[s % kRing][j]), __builtin_bit_cast(bf16x8, fa[s & 1][i]),
               acc[j][i], 0, 0, 0);
+      }
       if (kP1 && s < KK) p1_mfma(hacc, wmq[s % kRing], fl[s & 1]);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -981,6 +1103,114 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   {
     f32x16 none;
     phase2(last, hid + (last & 1) * (kMlpRows * kMlpHidRow), none, std::false_type{});
+  }
+
+  if constexpr (MODE != kMlpRaw) {
+    // ---- Reduce: bias, per-row LayerNorm moments over the D columns (in-lane,
+    // across the lane halves, across the waves; mean first, then the centred
+    // squares), then per group of K rows out = gamma . sum_r w_r (x_r - mean_r)
+    // rstd_r + beta . sum_r w_r.  Rows of weight 0 add exactly 0.
+    const int r32 = lane & 31, h4 = 4 * (lane >> 5);
+    float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < TNB; ++j) {
+      if (RAGGED && j >= nb) break;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 bv = *reinterpret_cast<const float4*>(&rd.b2[dw0 + 32 * j + 8 * q + h4]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          acc[j][i][4 * q] += bv.x;
+          acc[j][i][4 * q + 1] += bv.y;
+          acc[j][i][4 * q + 2] += bv.z;
+          acc[j][i][4 * q + 3] += bv.w;
+          sum[i] += (acc[j][i][4 * q] + acc[j][i][4 * q + 1]) +
+                    (acc[j][i][4 * q + 2] + acc[j][i][4 * q + 3]);
+        }
+      }
+    }
+    const float inv_d = 1.0f / static_cast<float>(mp.D);
+    float mean[2], scale[2];
+    auto across = [&](int which, float (&v)[2]) {  // the rows' sums over all waves
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v[i] = swap32_sum(v[i]);
+        if (lane < 32) rd.red[which][wave][32 * i + lane] = v[i];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v[i] = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kMlpWaves; ++w) v[i] += rd.red[which][w][32 * i + r32];
+      }
+    };
+    across(0, sum);  // (its barrier also ends the main loop's use of the LDS)
+    float sq[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      mean[i] = sum[i] * inv_d;
+#pragma unroll
+      for (int j = 0; j < TNB; ++j) {
+        if (RAGGED && j >= nb) break;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          acc[j][i][e] -= mean[i];
+          sq[i] = fmaf(acc[j][i][e], acc[j][i][e], sq[i]);
+        }
+      }
+    }
+    across(1, sq);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float w = rd.weight[32 * i + r32];
+      scale[i] = w * rsqrtf(sq[i] * inv_d + mp.eps);
+      if (w == 0.0f) {
+#pragma unroll
+        for (int j = 0; j < TNB; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.0f;
+        scale[i] = 0.0f;
+      }
+    }
+    // 32 columns at a time: the wave's 64 rows restaged, then a lane sums the K
+    // rows of (group, four columns).
+    unsigned char* st = smem + wave * (kMlpRows * kMlpStageRow);
+    const int K = p.K, groups = tile_rows / K;
+    const int64_t g0 = r0 / K, gall = p.rows / K;
+#pragma unroll
+    for (int j = 0; j < TNB; ++j) {
+      if (RAGGED && j >= nb) break;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(st + (32 * i + r32) * kMlpStageRow + (8 * q + h4) * 4) =
+              make_float4(acc[j][i][4 * q] * scale[i], acc[j][i][4 * q + 1] * scale[i],
+                          acc[j][i][4 * q + 2] * scale[i], acc[j][i][4 * q + 3] * scale[i]);
+      wave_sync();
+      const int quad = lane & 7, col = dw0 + 32 * j + 4 * quad;
+      const float4 ga = *reinterpret_cast<const float4*>(&rd.gamma[col]);
+      const float4 be = *reinterpret_cast<const float4*>(&rd.beta[col]);
+      for (int g = lane >> 3; g < groups; g += 8) {
+        if (g0 + g >= gall) break;
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float ws = 0.0f;
+        for (int kk = 0; kk < K; ++kk) {
+          const float4 x = *reinterpret_cast<const float4*>(st + (g * K + kk) * kMlpStageRow + 16 * quad);
+          v.x += x.x;
+          v.y += x.y;
+          v.z += x.z;
+          v.w += x.w;
+          ws += rd.weight[g * K + kk];
+        }
+        *reinterpret_cast<float4*>(mp.out + (g0 + g) * mp.D + col) =
+            make_float4(fmaf(ga.x, v.x, be.x * ws), fmaf(ga.y, v.y, be.y * ws),
+                        fmaf(ga.z, v.z, be.z * ws), fmaf(ga.w, v.w, be.w * ws));
+      }
+      wave_sync();
+    }
+    return;
   }
 
   // ---- Output: acc[j][i] holds raw[row 32i + (lane & 31)][columns dw0 + 32j +
@@ -2380,19 +2610,20 @@ bool mlp_fits_shape(int64_t R, int64_t H, int64_t D) {
          (D == 256 || D == 512 || D == 768);
 }
 
-template <int R, int TNB>
+template <int R, int TNB, int MODE = kMlpRaw, bool RAGGED = false>
 hipError_t launch_mlp_rt(const MlpParams& mp, hipStream_t stream) {
-  constexpr size_t lds = mlp_lds_bytes<R, TNB>();
+  constexpr size_t lds = mlp_lds_bytes<R, TNB, MODE>();
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&relation_mlp_kernel<R, TNB>),
+      reinterpret_cast<const void*>(&relation_mlp_kernel<R, TNB, MODE, RAGGED>),
       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   if (attr != hipSuccess) {
     set_error("relation_hidden_linear_seq: cannot reserve %zu bytes of LDS: %s", lds,
               hipGetErrorString(attr));
     return attr;
   }
-  const int64_t tiles = (mp.h.rows + kMlpRows - 1) / kMlpRows;
-  hipLaunchKernelGGL((relation_mlp_kernel<R, TNB>), dim3(static_cast<unsigned>(tiles)),
+  const int rows = MODE == kMlpRaw ? kMlpRows : mp.tile_rows;
+  const int64_t tiles = (mp.h.rows + rows - 1) / rows;
+  hipLaunchKernelGGL((relation_mlp_kernel<R, TNB, MODE, RAGGED>), dim3(static_cast<unsigned>(tiles)),
                      dim3(kMlpThreads), lds, stream, mp);
   return launch_status("relation_hidden_linear_seq");
 }
@@ -2402,6 +2633,22 @@ hipError_t launch_mlp_r(const MlpParams& mp, hipStream_t stream) {
   if (mp.D == 256) return launch_mlp_rt<R, 1>(mp, stream);
   if (mp.D == 512) return launch_mlp_rt<R, 2>(mp, stream);
   return launch_mlp_rt<R, 3>(mp, stream);
+}
+
+// Reduce forms: any d_model that is a multiple of 32 up to 768.
+template <int R, int MODE>
+hipError_t launch_mlp_reduce(const MlpParams& mp, hipStream_t stream) {
+  const bool even = mp.D % 256 == 0;
+  if (mp.D <= 256)
+    return even ? launch_mlp_rt<R, 1, MODE>(mp, stream) : launch_mlp_rt<R, 1, MODE, true>(mp, stream);
+  if (mp.D <= 512)
+    return even ? launch_mlp_rt<R, 2, MODE>(mp, stream) : launch_mlp_rt<R, 2, MODE, true>(mp, stream);
+  return even ? launch_mlp_rt<R, 3, MODE>(mp, stream) : launch_mlp_rt<R, 3, MODE, true>(mp, stream);
+}
+
+bool mlp_reduce_fits_shape(int64_t K, int64_t R, int64_t H, int64_t D) {
+  return (R == 64 || R == 128) && H > 0 && H % kMlpChunk == 0 && H <= (1 << 20) && D >= 32 &&
+         D <= kMlpMaxD && D % 32 == 0 && K >= 1 && K <= kMlpMaxK;
 }
 
 }  // namespace
@@ -2418,6 +2665,24 @@ __global__ void mfma_fragments_kernel(const uint16_t* __restrict__ w, uint16_t* 
   const int64_t nb = frag / kg, g = frag - nb * kg;
   const int64_t n = 32 * nb + (lane & 31), k = 16 * g + 8 * (lane >> 5);
   *reinterpret_cast<uint4*>(out + 8 * i) = *reinterpret_cast<const uint4*>(w + n * K + k);
+}
+
+// Two row-major weights ([N, K] each) in fragment order, one after the other.
+__global__ void mfma_fragments2_kernel(const uint16_t* __restrict__ w0, int64_t N0, int64_t K0,
+                                       const uint16_t* __restrict__ w1, int64_t N1, int64_t K1,
+                                       uint16_t* __restrict__ out) {
+  int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;  // one 16-byte piece
+  const int64_t n0 = N0 * K0 / 8;
+  const bool second = i >= n0;
+  const uint16_t* w = second ? w1 : w0;
+  const int64_t K = second ? K1 : K0, at = i;
+  i = second ? i - n0 : i;
+  if (at >= n0 + N1 * K1 / 8) return;
+  const int64_t lane = i & 63, frag = i >> 6;
+  const int64_t kg = K / 16;
+  const int64_t nb = frag / kg, g = frag - nb * kg;
+  const int64_t n = 32 * nb + (lane & 31), k = 16 * g + 8 * (lane >> 5);
+  *reinterpret_cast<uint4*>(out + 8 * at) = *reinterpret_cast<const uint4*>(w + n * K + k);
 }
 
 extern "C" hipError_t rlm_mfma_fragments(const rlm_tensor* weight, const rlm_tensor* out,
@@ -3007,4 +3272,163 @@ extern "C" hipError_t rlm_relation_linear_norm_reduce_output_noalloc(
       hidden, second_weight, second_bias, partner_scores, norm_weight, norm_bias, position,
       norm_eps, query, mix_logit, output_weight, output_bias, output_eps, &part, out_context,
       out_final, stream);
+}
+
+namespace rlm {
+namespace {
+// [D, H] of a second weight given row-major or in fragment order.
+bool second_dims(const rlm_tensor* t, int64_t& D, int64_t& H) {
+  if (t->ndim != 2) return frag_dims(t, D, H);
+  D = t->shape[0];
+  H = t->shape[1];
+  return true;
+}
+}  // namespace
+}  // namespace rlm
+
+extern "C" int rlm_relation_mlp_reduce_seq_fits(const rlm_tensor* expanded_cache,
+                                                const rlm_tensor* operand_cache,
+                                                const rlm_tensor* partner_index,
+                                                const rlm_tensor* product_weight,
+                                                const rlm_tensor* second_weight) {
+  for (const rlm_tensor* t : {expanded_cache, operand_cache, partner_index, product_weight,
+                              second_weight})
+    if (t == nullptr) return 0;
+  if (operand_cache->ndim != 3 || expanded_cache->ndim != 3 || partner_index->ndim != 3 ||
+      product_weight->ndim != 2)
+    return 0;
+  for (const rlm_tensor* t : {expanded_cache, operand_cache, product_weight, second_weight}) {
+    if (t->dtype != RLM_BF16 || (reinterpret_cast<uintptr_t>(t->data) & 15u) != 0) return 0;
+    int64_t bytes = 2;
+    for (int i = 0; i < t->ndim; ++i) bytes *= t->shape[i];
+    if (bytes >= (int64_t(1) << 31)) return 0;
+  }
+  const int64_t R = operand_cache->shape[2], H = product_weight->shape[0];
+  int64_t D, H2;
+  if (!second_dims(second_weight, D, H2) || product_weight->shape[1] != R || H2 != H ||
+      expanded_cache->shape[2] != 2 * H)
+    return 0;
+  return mlp_reduce_fits_shape(partner_index->shape[2], R, H, D) ? 1 : 0;
+}
+
+extern "C" hipError_t rlm_relation_mlp_reduce_seq(
+    const rlm_tensor* expanded_cache, const rlm_tensor* operand_cache,
+    const rlm_tensor* anchor_index, const rlm_tensor* partner_index,
+    const rlm_tensor* product_weight, const rlm_tensor* second_weight,
+    const rlm_tensor* second_bias, const rlm_tensor* partner_scores,
+    const rlm_tensor* norm_weight, const rlm_tensor* norm_bias, const rlm_tensor* positions,
+    double norm_eps, const rlm_tensor* workspace, const rlm_tensor* out, hipStream_t stream) {
+  clear_error();
+  const char* what = "relation_mlp_reduce_seq";
+  RLM_TRY(check_tensor(operand_cache, "operand_cache", 3));
+  RLM_TRY(check_tensor(expanded_cache, "expanded_cache", 3));
+  RLM_TRY(check_tensor(anchor_index, "anchor_index", 2));
+  RLM_TRY(check_tensor(partner_index, "partner_index", 3));
+  RLM_TRY(check_tensor(product_weight, "product_weight", 2));
+  RLM_REQUIRE(second_weight != nullptr, "second_weight: missing tensor");
+  const bool frag = second_weight->ndim == 4;
+  RLM_TRY(check_tensor(second_weight, "second_weight", frag ? 4 : 2));
+  RLM_REQUIRE(rlm_relation_mlp_reduce_seq_fits(expanded_cache, operand_cache, partner_index,
+                                               product_weight, second_weight),
+              "%s: needs bf16 caches and weights (16-byte aligned, under 2 GiB), relation dim 64 "
+              "or 128, a hidden dim that is a multiple of %d, d_model a multiple of 32 up to %d "
+              "and at most %d partners",
+              what, kMlpChunk, kMlpMaxD, kMlpMaxK);
+  const int64_t B = operand_cache->shape[0], T = operand_cache->shape[1];
+  const int64_t R = operand_cache->shape[2], H = product_weight->shape[0];
+  int64_t D, H2;
+  second_dims(second_weight, D, H2);
+  RLM_TRY(check_dim(expanded_cache, "expanded_cache", 0, B));
+  RLM_TRY(check_dim(expanded_cache, "expanded_cache", 1, T));
+  RLM_REQUIRE(is_index_dtype(anchor_index->dtype) && is_index_dtype(partner_index->dtype),
+              "anchor_index/partner_index must be int32 or int64");
+  RLM_TRY(check_dim(anchor_index, "anchor_index", 0, B));
+  RLM_TRY(check_dim(partner_index, "partner_index", 0, B));
+  const int64_t Tq = anchor_index->shape[1], K = partner_index->shape[2];
+  RLM_TRY(check_dim(partner_index, "partner_index", 1, Tq));
+  for (const auto& v : {std::make_pair(second_bias, "second_bias"),
+                        std::make_pair(norm_weight, "norm_weight"),
+                        std::make_pair(norm_bias, "norm_bias")}) {
+    RLM_TRY(check_tensor(v.first, v.second, 1));
+    RLM_TRY(check_dtype_float(v.first, v.second));
+    RLM_TRY(check_dim(v.first, v.second, 0, D));
+  }
+  RLM_TRY(check_tensor(partner_scores, "partner_scores", 3));
+  RLM_TRY(check_dtype_is(partner_scores, "partner_scores", RLM_F32));
+  RLM_TRY(check_dim(partner_scores, "partner_scores", 0, B));
+  RLM_TRY(check_dim(partner_scores, "partner_scores", 1, Tq));
+  RLM_TRY(check_dim(partner_scores, "partner_scores", 2, K));
+  RLM_TRY(check_tensor(workspace, "workspace", 1));
+  RLM_TRY(check_dtype_is(workspace, "workspace", RLM_BF16));
+  const int64_t packed = H * R + (frag ? 0 : D * H);
+  RLM_REQUIRE(workspace->shape[0] >= packed &&
+                  (reinterpret_cast<uintptr_t>(workspace->data) & 15u) == 0,
+              "%s: the workspace holds the row-major weights (%lld elements), 16-byte aligned",
+              what, (long long)packed);
+  RLM_TRY(check_tensor(out, "out", 3));
+  RLM_TRY(check_dtype_is(out, "out", RLM_F32));
+  RLM_TRY(check_dim(out, "out", 0, B));
+  RLM_TRY(check_dim(out, "out", 1, Tq));
+  RLM_TRY(check_dim(out, "out", 2, D));
+  RLM_REQUIRE((reinterpret_cast<uintptr_t>(out->data) & 15u) == 0, "%s: out must be 16-byte aligned",
+              what);
+  MlpParams mp{};
+  RLM_REQUIRE(positions != nullptr && is_index_dtype(positions->dtype),
+              "positions: expected an int32/int64 tensor");
+  if (positions->ndim == 1) {
+    RLM_TRY(check_tensor(positions, "positions", 1));
+    RLM_TRY(check_dim(positions, "positions", 0, Tq));
+    mp.pos_sb = 0;
+  } else {
+    RLM_TRY(check_tensor(positions, "positions", 2));
+    RLM_TRY(check_dim(positions, "positions", 0, B));
+    RLM_TRY(check_dim(positions, "positions", 1, Tq));
+    mp.pos_sb = Tq;
+  }
+  mp.pos_sq = 1;
+  mp.tile_rows = static_cast<int>(kMlpRows / K * K);
+  const int64_t rows = B * Tq * K;
+  RLM_REQUIRE((rows + mp.tile_rows - 1) / mp.tile_rows <= 0x7fffffff, "%s: too many relation rows", what);
+  if (rows == 0) return hipSuccess;
+  uint16_t* frags = static_cast<uint16_t*>(workspace->data);
+  const int64_t pieces = packed / 8;
+  hipLaunchKernelGGL(mfma_fragments2_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)),
+                     dim3(256), 0, stream, static_cast<const uint16_t*>(product_weight->data), H, R,
+                     static_cast<const uint16_t*>(second_weight->data), frag ? 0 : D, H, frags);
+  RLM_REQUIRE(launch_status(what) == hipSuccess, "%s: packing launch failed", what);
+  HiddenParams& p = mp.h;
+  p.B = B;
+  p.Tq = Tq;
+  p.T = T;
+  p.R = static_cast<int>(R);
+  p.H = static_cast<int>(H);
+  p.K = static_cast<int>(K);
+  p.rows = rows;
+  p.expanded = expanded_cache->data;
+  p.expanded_out = expanded_cache->data;
+  p.operand = operand_cache->data;
+  p.anchor = anchor_index->data;
+  p.partner = partner_index->data;
+  p.index_dtype_a = anchor_index->dtype;
+  p.index_dtype_p = partner_index->dtype;
+  p.wm = frags;
+  p.expanded_bytes = static_cast<uint32_t>(B * T * 2 * H * 2);
+  p.operand_bytes = static_cast<uint32_t>(B * T * R * 2);
+  p.wm_bytes = static_cast<uint32_t>(H * R * 2);
+  mp.w2 = frag ? second_weight->data : frags + H * R;
+  mp.w2_bytes = static_cast<uint32_t>(D * H * 2);
+  mp.out = static_cast<float*>(out->data);
+  mp.D = static_cast<int>(D);
+  mp.b2 = second_bias->data;
+  mp.b2_dtype = second_bias->dtype;
+  mp.gamma = norm_weight->data;
+  mp.gamma_dtype = norm_weight->dtype;
+  mp.beta = norm_bias->data;
+  mp.beta_dtype = norm_bias->dtype;
+  mp.eps = static_cast<float>(norm_eps);
+  mp.scores = static_cast<const float*>(partner_scores->data);
+  mp.pos = positions->data;
+  mp.pos_dtype = positions->dtype;
+  return R == 128 ? launch_mlp_reduce<128, kMlpQueries>(mp, stream)
+                  : launch_mlp_reduce<64, kMlpQueries>(mp, stream);
 }

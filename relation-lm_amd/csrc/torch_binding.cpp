@@ -815,6 +815,29 @@ std::tuple<at::Tensor, at::Tensor> relation_hidden_linear_norm_reduce_output(
 }
 
 
+// Whether the relation MLP kernel with the norm-reduce as its epilogue (64-row
+// tiles, plus a launch that packs the weights) is the faster form of the relation
+// reduce.
+//   Against the fused kernel (128-row tiles, K padded to a power of two): one tile
+//   per CU at a time, a 64-row round about 0.6 of a 128-row one.  D=512: B=8 T=512
+//   K=8 H=512 (2 rounds / 1) 43.8 / 34.3 us, B=8 T=2048 H=1024 (8 / 4) 261 / 256;
+//   B=4 T=256 K=8 D=256 H=1024 (1 / 1) 29.6 / 43.5, B=5 T=1728 K=5 D=384 H=512
+//   (3 / 3) 62 / 91.
+//   Against the three ops (other d_model): its tiles' chunk loop is a chain of
+//   H / 128 steps however few tiles there are.  H=2304 D=576: 768 rows 57 / 27 us,
+//   1024 58 / 37, 2048 58 / 82, 28672 134 / 386; H=512 D=320: 512 rows 18.6 / 17.4.
+bool mlp_reduce_faster(const at::Tensor& partner_index, bool fused_fits) {
+  const int64_t queries = partner_index.size(0) * partner_index.size(1);
+  const int64_t K = partner_index.size(2);
+  if (K < 1 || K > 16) return false;
+  if (!fused_fits) return queries * K >= 1536;
+  int64_t padded = 1;
+  while (padded < K) padded *= 2;
+  const int64_t rounds64 = (queries + (64 / K) * 256 - 1) / ((64 / K) * 256);
+  const int64_t rounds128 = (queries * padded + 128 * 256 - 1) / (128 * 256);
+  return 5 * rounds128 > 3 * rounds64;
+}
+
 at::Tensor relation_reduce_fused_seq(const at::Tensor& expanded_cache,
                                      const at::Tensor& operand_cache,
                                      const at::Tensor& anchor_index,
@@ -841,12 +864,30 @@ at::Tensor relation_reduce_fused_seq(const at::Tensor& expanded_cache,
     const rlm_tensor pi = desc(partner_index, "partner_index");
     const rlm_tensor wm = desc(product_weight, "product_weight");
     const rlm_tensor w2 = desc(second_weight, "second_weight");
-    if (!rlm_relation_reduce_fused_seq_fits(&e, &o, &pi, &wm, &w2)) {
-      TORCH_CHECK(!frag, op, ": a second_weight in fragment order needs the fused kernel's "
-                  "shapes (bf16, d_model 128/256/384/512, K <= 16, relation dim 32/64/128); "
-                  "pass the [D,H] weight for other shapes");
-      // Shapes or dtypes the fused kernel does not take (fp32, d_model 576, ...):
-      // the same result from the three-op chain it fuses, every step on HIP.
+    const bool fits = rlm_relation_reduce_fused_seq_fits(&e, &o, &pi, &wm, &w2) != 0;
+    TORCH_CHECK(fits || !frag, op, ": a second_weight in fragment order needs the fused kernel's "
+                "shapes (bf16, d_model 128/256/384/512, K <= 16, relation dim 32/64/128); "
+                "pass the [D,H] weight for other shapes");
+    if (mlp_reduce_faster(partner_index, fits) &&
+        rlm_relation_mlp_reduce_seq_fits(&e, &o, &pi, &wm, &w2)) {
+      at::Tensor out = at::empty({partner_index.size(0), partner_index.size(1), d_model},
+                                 f32(operand_cache));
+      at::Tensor workspace = at::empty(
+          {product_weight.numel() + (frag ? 0 : second_weight.numel())}, operand_cache.options());
+      const rlm_tensor ai = desc(anchor_index, "anchor_index");
+      const rlm_tensor b2 = desc(second_bias, "second_bias");
+      const rlm_tensor ps = desc(partner_scores, "partner_scores");
+      const rlm_tensor nw = desc(norm_weight, "norm_weight"), nb = desc(norm_bias, "norm_bias");
+      const rlm_tensor po = desc(positions, "positions"), ws = desc(workspace, "workspace");
+      const rlm_tensor oo = desc(out, "out");
+      check(rlm_relation_mlp_reduce_seq(&e, &o, &ai, &pi, &wm, &w2, &b2, &ps, &nw, &nb, &po,
+                                        norm_eps, &ws, &oo, stream),
+            op);
+      return out;
+    }
+    if (!fits) {
+      // Shapes or dtypes neither kernel takes (fp32, K > 16, ...): the same result
+      // from the three-op chain, every step on HIP.
       const at::Tensor hidden = relation_hidden_cached_seq(expanded_cache, operand_cache,
                                                            anchor_index, partner_index,
                                                            product_weight);
