@@ -314,6 +314,32 @@ int rlm_relation_mlp_reduce_seq_fits(const rlm_tensor* expanded_cache,
                                      const rlm_tensor* product_weight,
                                      const rlm_tensor* second_weight);
 
+/*
+ * The multi-anchor block after its selection (multi_relation_blocks.py:148-178):
+ * relation MLP with its LayerNorm, partner and slot mixing, residual gate -- the
+ * calls rlm_relation_hidden_linear_seq and rlm_multi_relation_reduce_seq without
+ * the [B,Tq,S,K,D] rows between them: a slot's weighted sum leaves the MLP kernel
+ * instead, and a second launch adds a query's slots.
+ *   caches and weights as rlm_relation_hidden_linear_seq (in fragment order);
+ *   anchor_index [B,Tq*S], partner_index [B,Tq*S,K], partner_scores f32
+ *   [B,Tq,S,K], second_bias / norm_weight / norm_bias [D], slot_mix_logits [S],
+ *   residual_gate [] and hidden [B,Tq,D] (any float dtype), positions [Tq] or
+ *   [B,Tq]; workspace f32 of rlm_relation_block_seq_workspace(B*Tq*S, K, D)
+ *   elements, 16-byte aligned.
+ * Outputs: out [B,Tq,D] in hidden's dtype; out_context f32 [B,Tq,D] or NULL.
+ * Shapes: rlm_relation_hidden_linear_seq's, K in 1..64.
+ */
+hipError_t rlm_relation_block_seq(
+    const rlm_tensor* expanded_cache, const rlm_tensor* operand_cache,
+    const rlm_tensor* anchor_index, const rlm_tensor* partner_index,
+    const rlm_tensor* product_weight, const rlm_tensor* second_weight,
+    const rlm_tensor* second_bias, const rlm_tensor* partner_scores,
+    const rlm_tensor* norm_weight, const rlm_tensor* norm_bias,
+    const rlm_tensor* slot_mix_logits, const rlm_tensor* residual_gate, const rlm_tensor* hidden,
+    const rlm_tensor* positions, double norm_eps, const rlm_tensor* workspace,
+    const rlm_tensor* out, const rlm_tensor* out_context, hipStream_t stream);
+int64_t rlm_relation_block_seq_workspace(int64_t groups, int64_t partners, int64_t d_model);
+
 /* 1 if rlm_relation_hidden_linear_seq takes these tensors (dtypes, shapes,
  * alignment; the weights in fragment order), else 0. */
 int rlm_relation_hidden_linear_seq_fits(const rlm_tensor* expanded_cache,

@@ -1170,6 +1170,54 @@ void multi_relation_reduce_seq_out(const at::Tensor& raw, const at::Tensor& part
         op);
 }
 
+// The multi-anchor block after its selection, into caller tensors (out: hidden's
+// shape and dtype; out_context: fp32, when given).
+void relation_block_seq_out(const at::Tensor& expanded_cache, const at::Tensor& operand_cache,
+                            const at::Tensor& anchor_index, const at::Tensor& partner_index,
+                            const at::Tensor& product_weight, const at::Tensor& second_weight,
+                            const at::Tensor& second_bias, const at::Tensor& partner_scores,
+                            const at::Tensor& norm_weight, const at::Tensor& norm_bias,
+                            const at::Tensor& slot_mix_logits, const at::Tensor& residual_gate,
+                            const at::Tensor& hidden, const at::Tensor& positions,
+                            double norm_eps, at::Tensor& out,
+                            const c10::optional<at::Tensor>& context) {
+  const char* op = "relation_lm_block::relation_block_seq_out";
+  const at::Tensor ctx = context.has_value() ? *context : at::Tensor();
+  c10::DeviceGuard guard(hidden.device());
+  hipStream_t stream = device_stream(
+      op, {&expanded_cache, &operand_cache, &anchor_index, &partner_index, &product_weight,
+           &second_weight, &second_bias, &partner_scores, &norm_weight, &norm_bias,
+           &slot_mix_logits, &residual_gate, &hidden, &positions, &out, &ctx});
+  TORCH_CHECK(partner_scores.dim() == 4 && hidden.dim() == 3, op,
+              ": partner_scores must be [B,Tq,S,K] and hidden [B,Tq,D]");
+  const int64_t groups = partner_scores.size(0) * partner_scores.size(1) * partner_scores.size(2);
+  at::Tensor workspace = at::empty(
+      {rlm_relation_block_seq_workspace(groups, partner_scores.size(3), hidden.size(2))},
+      f32(hidden));
+  rlm_tensor d[17] = {desc(expanded_cache, "expanded_cache"),
+                      desc(operand_cache, "operand_cache"),
+                      desc(anchor_index, "anchor_index"),
+                      desc(partner_index, "partner_index"),
+                      desc(product_weight, "product_weight"),
+                      desc(second_weight, "second_weight"),
+                      desc(second_bias, "second_bias"),
+                      desc(partner_scores, "partner_scores"),
+                      desc(norm_weight, "norm_weight"),
+                      desc(norm_bias, "norm_bias"),
+                      desc(slot_mix_logits, "slot_mix_logits"),
+                      desc(residual_gate, "residual_gate"),
+                      desc(hidden, "hidden"),
+                      desc(positions, "positions"),
+                      desc(workspace, "workspace"),
+                      desc(out, "out"),
+                      rlm_tensor{}};
+  if (ctx.defined()) d[16] = desc(ctx, "context");
+  check(rlm_relation_block_seq(&d[0], &d[1], &d[2], &d[3], &d[4], &d[5], &d[6], &d[7], &d[8],
+                               &d[9], &d[10], &d[11], &d[12], &d[13], norm_eps, &d[14], &d[15],
+                               ctx.defined() ? &d[16] : nullptr, stream),
+        op);
+}
+
 at::Tensor layer_norm(const at::Tensor& input, const at::Tensor& weight, const at::Tensor& bias,
                       double eps) {
   const char* op = "relation_lm::layer_norm";
@@ -1351,6 +1399,16 @@ TORCH_LIBRARY(relation_lm, m) {
   m.def("block_statistics(Tensor keys, SymInt block_size) -> (Tensor, Tensor)");
 }
 
+// Steps of the block modules that are no operators of their own.
+TORCH_LIBRARY(relation_lm_block, m) {
+  m.def(
+      "relation_block_seq_out(Tensor expanded_cache, Tensor operand_cache, Tensor anchor_index, "
+      "Tensor partner_index, Tensor product_weight, Tensor second_weight, Tensor second_bias, "
+      "Tensor partner_scores, Tensor norm_weight, Tensor norm_bias, Tensor slot_mix_logits, "
+      "Tensor residual_gate, Tensor hidden, Tensor positions, float norm_eps, Tensor(a!) out, "
+      "Tensor(b!)? context=None) -> ()");
+}
+
 TORCH_LIBRARY(relationlex, m) {
   m.def(
       "anchor_select(Tensor anchor_query, Tensor anchor_keys, Tensor router_query, Tensor "
@@ -1407,6 +1465,10 @@ TORCH_LIBRARY_IMPL(relation_lm, CPU, m) {
                 "relation_lm::packed_sparse_cache_projection: memory and weight must share a device");
     return at::linear(memory, weight);
   });
+}
+
+TORCH_LIBRARY_IMPL(relation_lm_block, CUDA, m) {
+  m.impl("relation_block_seq_out", TORCH_FN(relation_block_seq_out));
 }
 
 TORCH_LIBRARY_IMPL(relationlex, CUDA, m) {

@@ -165,6 +165,12 @@ def _register_fakes() -> None:
           positions, norm_eps, raw_bias, out, context=None):
         return None
 
+    @torch.library.register_fake("relation_lm_block::relation_block_seq_out")
+    def _(expanded_cache, operand_cache, anchor_index, partner_index, product_weight,
+          second_weight, second_bias, partner_scores, norm_weight, norm_bias, slot_mix_logits,
+          residual_gate, hidden, positions, norm_eps, out, context=None):
+        return None
+
     def fake_norm_output(raw, partner_scores, norm_weight, norm_bias, position, norm_eps, query,
                          mix_logit, output_weight, output_bias, output_eps):
         shape = tuple(raw.shape[:-2]) + (raw.shape[-1],)

@@ -11,15 +11,14 @@ multi-anchor selection (local window plus the top blocks of a block router,
   projections of hidden / memory  relation_lm::relation_linear (MFMA)
   router block statistics         relation_lm::block_statistics
   distinct anchors, partners      relation_lm::multi_relation_select_seq
-  relation MLP Linear -> GELU     relation_lm::relation_hidden_linear_seq_out: one
-    -> Linear (bias-free)           kernel (factorized first Linear: operand cache,
-                                    expanded cache = [W_a+W_d; W_p-W_d] op + [b; 0];
-                                    the bf16 hidden stays on chip; fp32 output)
-    other shapes                    relation_lm::relation_hidden_cached_seq_out, then
-                                    relation_lm::relation_linear (MFMA DMA-tile GEMM)
-  second Linear's bias, LayerNorm, relation_lm::multi_relation_reduce_seq
-    partner softmax, slot mix,
-    residual gate
+  relation MLP Linear -> GELU     relation_lm_block::relation_block_seq_out: one
+    -> Linear -> LayerNorm,         kernel up to the slots' sums (factorized first
+    partner softmax and sum,        Linear: operand cache, expanded cache =
+    slot mix, residual gate         [W_a+W_d; W_p-W_d] op + [b; 0]; hidden and rows
+                                    stay on chip), one for the slot mix and gate
+    other shapes                    relation_lm::relation_hidden_cached_seq_out,
+                                    relation_lm::relation_linear (MFMA DMA-tile GEMM),
+                                    relation_lm::multi_relation_reduce_seq
   final_norm (stack)              relation_lm::layer_norm
 
 When the sequence is no longer than the local window every causal position is
@@ -49,6 +48,7 @@ from relation_lm.kernels.relation_reduce import (factor_relation_first_layer, mf
                                                  relation_hidden_linear_seq_fits)
 
 ops = torch.ops.relation_lm
+block_ops = torch.ops.relation_lm_block
 
 
 @dataclass
@@ -215,31 +215,26 @@ class MultiAnchorRelationBlock(nn.Module):
         mlp = self.relation_mlp
         output = torch.empty_like(hidden, memory_format=torch.contiguous_format)
         wm_frags, w2_frags = sel.get("product_weight_frags"), sel.get("second_weight_frags")
-        if wm_frags is not None and relation_hidden_linear_seq_fits(
-                sel["expanded_cache"], sel["operand_cache"], wm_frags, w2_frags):
-            # The hidden and the bias-free second Linear in one launch (the
-            # hidden never reaches memory); the second Linear's bias joins the
-            # rows as the slot reduce loads them.  Equal groups of batch rows,
-            # each group's fp32 rows below the 2 GiB a kernel addresses.
-            raw_bytes = length * h * k_count * d * 4
-            most = max(1, min(batch, (2**31 - 1) // raw_bytes))
+        if (wm_frags is not None and h * k_count <= 64
+                and relation_hidden_linear_seq_fits(sel["expanded_cache"], sel["operand_cache"],
+                                                    wm_frags, w2_frags)):
+            # The relation MLP with its LayerNorm and the slots' weighted sums in one
+            # launch (neither the hidden nor the rows reach memory), then the slot
+            # mix and the residual gate.  Equal groups of batch rows, each group's
+            # expanded cache and slot sums below the 2 GiB a kernel addresses.
+            row_bytes = length * max(2 * sel["expanded_cache"].shape[2], 4 * h * d)
+            most = max(1, min(batch, (2**31 - 1) // row_bytes))
             group = -(-batch // -(-batch // most))
-            raw = torch.empty((group, length * h, k_count, d), dtype=torch.float32,
-                              device=hidden.device)
             for b0 in range(0, batch, group):
                 b1 = min(batch, b0 + group)
                 n = b1 - b0
-                part = raw[:n]
-                ops.relation_hidden_linear_seq_out(
+                block_ops.relation_block_seq_out(
                     sel["expanded_cache"][b0:b1], sel["operand_cache"][b0:b1],
                     sel["anchor"][b0:b1].reshape(n, length * h),
                     sel["partner"][b0:b1].reshape(n, length * h, k_count), wm_frags, w2_frags,
-                    part)
-                ops.multi_relation_reduce_seq_out(
-                    part.view(n, length, h, k_count, d), sel["partner_score"][b0:b1],
-                    mlp[3].weight, mlp[3].bias, self.slot_mix_logits, self.residual_gate,
-                    hidden[b0:b1], sel["positions"], mlp[3].eps, mlp[2].bias, output[b0:b1],
-                    None if context is None else context[b0:b1])
+                    mlp[2].bias, sel["partner_score"][b0:b1], mlp[3].weight, mlp[3].bias,
+                    self.slot_mix_logits, self.residual_gate, hidden[b0:b1], sel["positions"],
+                    mlp[3].eps, output[b0:b1], None if context is None else context[b0:b1])
             return output
         # Other shapes: the hidden, then the second Linear.
         # The MLP hidden in the second Linear's operand dtype: a bf16 Linear
