@@ -14,8 +14,9 @@
 //                 tile per CU) on v_mfma_f32_32x32x16; A and W k-slices of 64 go
 //                 from global memory straight into LDS (two stages), the
 //                 output is restaged through LDS into whole row segments.
-//   split_kernel  (M > 64, fp32 A, few tiles) 32x32 tiles, the eight waves of a
-//                 workgroup split K, each through LDS stages of its own.
+//   split_kernel  (fp32 A, few tiles; K >= 1024 where M <= 64) 16x16 or 32x32
+//                 tiles, the eight waves of a workgroup split K, each through LDS
+//                 stages of its own.
 //   tile_kernel   (M > 64, the other cases: fp32 A, K % 64 != 0)
 //                 BMxBN workgroup tile (128x128 or 64x128), four
 //                 waves in 2x2, each a (BM/2)x(BN/2) grid of 16x16 MFMA tiles.
@@ -34,7 +35,7 @@
 //                 forms a 64x64 output tile as (W . A^T) so that a lane holds
 //                 four consecutive columns of a row (16-byte stores for fp32
 //                 output, 8-byte LDS staging then 16-byte row pieces for 16-bit).
-//   skinny_kernel (M <= 64)  decode shapes.  A workgroup owns one 16x16 output
+//   skinny_kernel (M <= 64, the other cases)  decode shapes.  A workgroup owns one 16x16 output
 //                 tile; its eight waves split K, each issuing the W and A
 //                 fragment loads of up to six 32-wide slices at once straight
 //                 from global memory in MFMA operand layout, and the partial
@@ -42,8 +43,9 @@
 //
 // fp32 weights (fp32 operands and accumulation throughout, so fp32 mode never
 // passes through reduced precision): split_kernel for few tiles and
-// dma_tile_kernel with 64x64 tiles otherwise, both on v_mfma_f32_32x32x2f32;
-// f32_skinny_kernel (M <= 32: fp32 FMA dot products split over a wave); and
+// dma_tile_kernel with 64x64 tiles otherwise, on v_mfma_f32_32x32x2f32 and
+// v_mfma_f32_16x16x4f32; f32_skinny_kernel (M <= 64 where split_kernel does not
+// fit: fp32 FMA dot products split over a wave); and
 // f32_tile_kernel (v_mfma_f32_16x16x4f32) for K % 32 != 0 or unaligned rows.
 #include "rlm_common.hpp"
 
@@ -997,40 +999,46 @@ __global__ void __launch_bounds__(WM * WN * kWave) dma_tile_kernel(const GemmPar
 // fp32 A, few output tiles: the waves of a workgroup split K
 // ---------------------------------------------------------------------------
 //
-// Decode batches (64 < M <= a few hundred rows of an fp32 hidden against a
-// 16-bit weight) and small fp32 problems have too few large tiles to fill the
-// chip, and a tile's K loop is then one long chain of load round trips (M = 192,
-// N = 576, K = 2304: 15 tiles of 64 x 128, 42 us).  Here a workgroup of eight
-// waves owns one 32 x 32 output tile and each wave takes every eighth 32-wide
-// chunk of K through its own LDS stages: LDS-DMA moves whole row segments (one
-// L1 access per 128-byte line; fragments loaded straight from global memory
-// touch a line per lane pair, and the L1 then takes 15 us on the shape above),
-// NS chunks in flight per wave, no barrier before the end.  The eight partial
-// tiles meet once in LDS and are added in wave order.  The product is W . A^T,
-// so a lane ends with four consecutive columns of a row.
+// Decode batches (an fp32 hidden against a 16-bit weight, M up to a few hundred
+// rows) and small fp32 problems have too few large tiles to fill the chip, and a
+// tile's K loop is then one long chain of load round trips (M = 192, N = 576,
+// K = 2304: 15 tiles of 64 x 128, 42 us).  Here a workgroup of eight waves owns
+// one TS x TS output tile (TS = 16 or 32: one MFMA's) and each wave takes every
+// eighth 32-wide chunk of K through its own LDS stages: LDS-DMA moves whole row
+// segments (one L1 access per 128-byte line; fragments loaded straight from
+// global memory touch a line per lane pair, and the L1 then takes 15 us on the
+// shape above), NS chunks in flight per wave, no barrier before the end.  The
+// eight partial tiles meet once in LDS and are added in wave order.  The product
+// is W . A^T, so a lane ends with four consecutive columns of a row.  fp32 MFMAs
+// bound the 32 x 32 tiles of an fp32 W (M = 24, N = 576, K = 2304: 144 of 64
+// cycles a wave, 11.7 us); 16 x 16 ones spread them over four times the CUs
+// (6.0 us).
 constexpr int kSplitWaves = 8;
 
-template <typename W>
+template <typename W, int TS>
 struct SplitForm {
   static constexpr int kWRow = 32 * static_cast<int>(sizeof(W));  // bytes of a W chunk row
-  static constexpr int kStage = 32 * 128 + 32 * kWRow;            // A and W of one chunk
+  static constexpr int kA = TS * 128;                             // bytes of a chunk of A
+  static constexpr int kStage = kA + TS * kWRow;                  // A and W of one chunk
   static constexpr int kLoads = kStage / 1024;                    // DMA instructions per chunk
-  static constexpr int NS = sizeof(W) == 2 ? 3 : 2;               // stages per wave
+  static constexpr int NS = TS == 16 ? 4 : sizeof(W) == 2 ? 3 : 2;  // stages per wave
   static constexpr size_t kLds = static_cast<size_t>(kSplitWaves) * NS * kStage;
 };
 
-template <typename W, typename TO>
+template <typename W, typename TO, int TS>
 __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmParams p) {
-  using F = SplitForm<W>;
+  using F = SplitForm<W, TS>;
+  static_assert(TS == 16 || TS == 32, "a tile is one MFMA's");
+  constexpr int kQuads = TS * TS / 256;  // four-element pieces of a lane's partial tile
   constexpr int NS = F::NS;
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int64_t tiles_n = (p.N + 31) / 32;
+  const int64_t tiles_n = (p.N + TS - 1) / TS;
   const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int64_t m0 = (tile / tiles_n) * 32;
-  const int64_t n0 = (tile % tiles_n) * 32;
+  const int64_t m0 = (tile / tiles_n) * TS;
+  const int64_t n0 = (tile % tiles_n) * TS;
   const rsrc_t ar = make_rsrc(p.a, p.a_bytes);
   const rsrc_t wr = make_rsrc(p.w, p.w_bytes);
   unsigned char* mine = smem + wave * (NS * F::kStage);
@@ -1040,16 +1048,17 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
   // DMA lane roles.  128-byte rows: eight lanes per row, LDS piece q of row r
   // holds piece q ^ dma_swz<64>(r); 64-byte rows: four, dma_swz<32>.  Rows past
   // M or N read zeros.
-  uint32_t a_off[4], w_off[F::kWRow / 32];
+  constexpr int kADma = TS / 8, kWDma = TS * F::kWRow / 1024;
+  uint32_t a_off[kADma], w_off[kWDma];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
+  for (int d = 0; d < kADma; ++d) {
     const int r = 8 * d + (lane >> 3);
     a_off[d] = m0 + r < p.M ? static_cast<uint32_t>((m0 + r) * p.lda * 4) +
                                   ((lane & 7) ^ dma_swz<64>(r & 15)) * 16u
                             : kNoOffset;
   }
 #pragma unroll
-  for (int d = 0; d < F::kWRow / 32; ++d) {
+  for (int d = 0; d < kWDma; ++d) {
     constexpr bool wide = sizeof(W) == 4;
     const int r = wide ? 8 * d + (lane >> 3) : 16 * d + (lane >> 2);
     const int q = wide ? (lane & 7) ^ dma_swz<64>(r & 15) : (lane & 3) ^ dma_swz<32>(r & 15);
@@ -1059,22 +1068,29 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
   auto issue = [&](int stage, int chunk) {
     const uint32_t st = lds0 + stage * F::kStage;
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
+    for (int d = 0; d < kADma; ++d)
       lds_dma16(ar, st + 1024u * d, a_off[d], static_cast<uint32_t>(chunk) * 128u);
 #pragma unroll
-    for (int d = 0; d < F::kWRow / 32; ++d)
-      lds_dma16(wr, st + 4096u + 1024u * d, w_off[d], static_cast<uint32_t>(chunk) * F::kWRow);
+    for (int d = 0; d < kWDma; ++d)
+      lds_dma16(wr, st + F::kA + 1024u * d, w_off[d], static_cast<uint32_t>(chunk) * F::kWRow);
   };
 
-  f32x16 acc;
+  // fp32: the steps of a chunk have their own sums (added pairwise at the end), so
+  // that no fp32 chain is longer than K / 64 products, as the lanes of
+  // f32_skinny_kernel keep it (K = 2304, N = 576, against fp64: one chain 1.4e-6).
+  typedef float acc_t __attribute__((ext_vector_type(4 * kQuads)));
+  constexpr int kAccs = sizeof(W) == 2 ? 1 : TS == 16 ? 8 : 4;
+  acc_t accs[kAccs];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+  for (int a = 0; a < kAccs; ++a)
+#pragma unroll
+    for (int e = 0; e < 4 * kQuads; ++e) accs[a][e] = 0.0f;
   const int chunks = static_cast<int>(p.K / 32);
   const int own = chunks > wave ? (chunks - wave + kSplitWaves - 1) / kSplitWaves : 0;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
     if (s < own) issue(s, wave + s * kSplitWaves);
-  const int r = lane & 31, h = lane >> 5;
+  const int r = lane & (TS - 1), h = lane / TS;  // row of the fragments, k-group
   const int sa = dma_swz<64>(r & 15), sw = sizeof(W) == 4 ? sa : dma_swz<32>(r & 15);
   int stage = 0;
   for (int i = 0; i < own; ++i) {
@@ -1085,8 +1101,22 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     const unsigned char* sta = mine + stage * F::kStage + r * 128;
-    const unsigned char* stw = mine + stage * F::kStage + 4096 + r * F::kWRow;
-    if constexpr (sizeof(W) == 4) {
+    const unsigned char* stw = mine + stage * F::kStage + F::kA + r * F::kWRow;
+    if constexpr (TS == 16 && sizeof(W) == 4) {
+      // Steps of four k: lane group h takes k = 16 g + 4 h + e of step (g, e).
+      f32x4 a[2], w[2];
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        a[g] = *reinterpret_cast<const f32x4*>(sta + 16 * ((4 * g + h) ^ sa));
+        w[g] = *reinterpret_cast<const f32x4*>(stw + 16 * ((4 * g + h) ^ sw));
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          accs[4 * g + e] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(w[g][e], a[g][e], accs[4 * g + e], 0, 0, 0);
+    } else if constexpr (sizeof(W) == 4) {
       u16x8 a[4], w[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -1094,19 +1124,21 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
         w[g] = *reinterpret_cast<const u16x8*>(stw + 16 * ((2 * g + h) ^ sw));
       }
 #pragma unroll
-      for (int g = 0; g < 4; ++g) acc = mfma32<W>(w[g], a[g], acc);
+      for (int g = 0; g < 4; ++g) accs[g] = mfma32<W>(w[g], a[g], accs[g]);
     } else {
-      f32x4 x[2][2];
-      u16x8 w[2];
+      // 16-bit W: eight k a lane, 2 (32 x 32: 16 k) or 4 (16 x 16: 32 k) lane groups.
+      constexpr int G = TS / 16, KG = 64 / TS;
+      f32x4 x[G][2];
+      u16x8 w[G];
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
+      for (int g = 0; g < G; ++g) {
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          x[g][e] = *reinterpret_cast<const f32x4*>(sta + 16 * ((4 * g + 2 * h + e) ^ sa));
-        w[g] = *reinterpret_cast<const u16x8*>(stw + 16 * ((2 * g + h) ^ sw));
+          x[g][e] = *reinterpret_cast<const f32x4*>(sta + 16 * ((2 * (KG * g + h) + e) ^ sa));
+        w[g] = *reinterpret_cast<const u16x8*>(stw + 16 * ((KG * g + h) ^ sw));
       }
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
+      for (int g = 0; g < G; ++g) {
         uint32_t a[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1114,7 +1146,9 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
           if constexpr (__is_same(W, bf16)) a[e] = pack_bf16x2(lo, hi);
           else a[e] = pack2(to_bits<W>(lo), to_bits<W>(hi));
         }
-        acc = mfma32<W>(w[g], __builtin_bit_cast(u16x8, make_uint4(a[0], a[1], a[2], a[3])), acc);
+        const u16x8 af = __builtin_bit_cast(u16x8, make_uint4(a[0], a[1], a[2], a[3]));
+        if constexpr (TS == 32) accs[0] = mfma32<W>(w[g], af, accs[0]);
+        else accs[0] = mfma16<W>(w[g], af, accs[0]);
       }
     }
     if (i + NS < own) {
@@ -1123,22 +1157,28 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
     }
     stage = stage + 1 == NS ? 0 : stage + 1;
   }
+#pragma unroll
+  for (int a = kAccs / 2; a > 0; a /= 2)
+#pragma unroll
+    for (int b = 0; b < a; ++b) accs[b] += accs[a + b];
+  const acc_t acc = accs[0];
   __syncthreads();  // every wave is done with its stages
   f32x4* part = reinterpret_cast<f32x4*>(smem);  // [wave][quad][lane]
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-    part[(wave * 4 + q) * kWave + lane] =
+  for (int q = 0; q < kQuads; ++q)
+    part[(wave * kQuads + q) * kWave + lane] =
         f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
   __syncthreads();
-  // Quad q of lane l holds columns 8q + 4 (l / 32) .. +3 of row l % 32.
+  // Quad q of lane l holds columns (256 / TS) q + 4 (l / TS) .. +3 of row l % TS.
   // Thread -> (row m, column quad nq), columns fastest: a row's pieces leave
   // side by side.
-  if (tid >= 256) return;
-  const int m = tid >> 3, nq = tid & 7;
-  const int at = (nq >> 1) * kWave + m + 32 * (nq & 1);
+  if (tid >= TS * TS / 4) return;
+  constexpr int kNq = TS / 4, kGroups = 64 / TS;  // column quads of a row, lane groups
+  const int m = tid / kNq, nq = tid % kNq;
+  const int at = nq / kGroups * kWave + m + TS * (nq % kGroups);
   f32x4 sum = part[at];
 #pragma unroll
-  for (int w = 1; w < kSplitWaves; ++w) sum += part[w * 4 * kWave + at];
+  for (int w = 1; w < kSplitWaves; ++w) sum += part[w * kQuads * kWave + at];
   const int64_t mm = m0 + m, n = n0 + 4 * nq;
   if (mm >= p.M) return;
   TO* out = static_cast<TO*>(p.out) + mm * p.ldo + n;
@@ -1155,20 +1195,33 @@ __global__ void __launch_bounds__(kSplitWaves * kWave) split_kernel(const GemmPa
   }
 }
 
-template <typename W, typename TO>
-hipError_t launch_split(const GemmParams& p, hipStream_t s) {
-  constexpr size_t lds = SplitForm<W>::kLds;
+template <typename W, typename TO, int TS>
+hipError_t launch_split_tile(const GemmParams& p, hipStream_t s) {
+  constexpr size_t lds = SplitForm<W, TS>::kLds;
   static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&split_kernel<W, TO>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&split_kernel<W, TO, TS>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   if (attr != hipSuccess) {
     set_error("linear: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr));
     return attr;
   }
-  const int64_t tiles = ((p.M + 31) / 32) * ((p.N + 31) / 32);
-  hipLaunchKernelGGL((split_kernel<W, TO>), dim3(static_cast<unsigned>(tiles)),
+  const int64_t tiles = ((p.M + TS - 1) / TS) * ((p.N + TS - 1) / TS);
+  hipLaunchKernelGGL((split_kernel<W, TO, TS>), dim3(static_cast<unsigned>(tiles)),
                      dim3(kSplitWaves * kWave), lds, s, p);
   return launch_status("linear");
+}
+
+inline int64_t tiles_of(const GemmParams& p, int64_t ts) {
+  return ((p.M + ts - 1) / ts) * ((p.N + ts - 1) / ts);
+}
+
+template <typename W, typename TO>
+hipError_t launch_split(const GemmParams& p, hipStream_t s) {
+  // 16 x 16 tiles while they are at most one per CU.  16 / 32, us, fp32 and bf16 W:
+  //   M=64 N=576 K=2304 (144)  6.1 / 11.8, 4.9 / 6.5     M=128 N=512 K=512 (256)  3.8 / 5.3, 3.5 / 4.0
+  //   M=128 N=576 K=2304 (288) 13.7 / 12.0, 8.4 / 6.6    M=256 N=512 K=512 (512)  6.0 / 5.5, 5.5 / 4.1
+  if (tiles_of(p, 16) <= 256) return launch_split_tile<W, TO, 16>(p, s);
+  return launch_split_tile<W, TO, 32>(p, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1354,22 +1407,22 @@ inline bool split_fits(const GemmParams& p) {
 template <typename TO>
 hipError_t launch_f32(const GemmParams& p, hipStream_t s) {
   // split / skinny / 64x64 DMA tiles / f32_tile, us:
-  //   M=1 N=512 K=576       5.6 / 4.6 / 12.7 / 42     M=4 N=4608 K=128  3.6 / 7.1 / 4.8 / 11.9
-  //   M=64 N=576 K=2304    12.0 / 14.8 / 44 / 198     M=128 N=2048 K=128  3.9 / - / 5.3 / 15
-  //   M=1024 N=256 K=1024   7.9 / - / 21.6 / 89       M=1024 N=512 K=512 (512 split tiles)  10.1 / - / 12.6 / 47
+  //   M=4 N=576 K=2304      6.0 / 9.0             M=1 N=512 K=576       3.6 / 4.4 / 12.7 / 42
+  //   M=24 N=576 K=2304     6.0 / 11.2            M=4 N=4608 K=128  3.6 / 7.1 / 4.8 / 11.9
+  //   M=64 N=576 K=2304     6.1 / 14.8 / 44 / 198     M=128 N=2048 K=128  3.8 / - / 5.3 / 15
+  //   M=1024 N=256 K=1024   7.8 / - / 21.6 / 89       M=1024 N=512 K=512 (512 split tiles)  10.1 / - / 12.6 / 47
   //   M=1024 N=2048 K=128  21.3 / - / 9.1 / 23        M=15360 N=512 K=512  126 / - / 79 / 231
-  const int64_t t32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+  const int64_t t32 = tiles_of(p, 32);
   const bool aligned = p.lda % 4 == 0 && (reinterpret_cast<uintptr_t>(p.a) & 15u) == 0 &&
                        (reinterpret_cast<uintptr_t>(p.w) & 15u) == 0;
-  const bool split = split_fits(p) && (t32 <= 256 || (t32 <= 512 && p.K >= 512));
-  if (p.M <= kSkinnyM && p.a_bytes != 0 && p.K % 4 == 0 && aligned &&
-      !(split && (p.M > 32 || p.K < 256))) {
+  if (split_fits(p) && (t32 <= 256 || (t32 <= 512 && p.K >= 512)))
+    return launch_split<float, TO>(p, s);
+  if (p.M <= kSkinnyM && p.a_bytes != 0 && p.K % 4 == 0 && aligned) {
     const dim3 grid(static_cast<unsigned>((p.N + 4 * kF32SkinnyCols - 1) / (4 * kF32SkinnyCols)),
                     static_cast<unsigned>((p.M + kF32SkinnyRows - 1) / kF32SkinnyRows));
     hipLaunchKernelGGL((f32_skinny_kernel<TO>), grid, dim3(256), 0, s, p);
     return launch_status("linear");
   }
-  if (split) return launch_split<float, TO>(p, s);
   constexpr int64_t kLimit = int64_t(1) << 31;
   if (aligned && p.K % 32 == 0 && (p.ldo * static_cast<int64_t>(sizeof(TO))) % 16 == 0 &&
       (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0 && 64 * p.lda * 4 < kLimit &&
@@ -1403,6 +1456,13 @@ bool dma_fits(const GemmParams& p) {
 
 template <typename TA, typename W, typename TO>
 hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
+  // An fp32 A with long rows: split / skinny, us: M=64 N=576 K=2304 4.9 / 8.4,
+  // M=4 N=576 K=2304 4.6 / 6.1, M=32 N=256 K=1024 3.8 / 5.8; M=8 N=1024 K=512
+  // 3.3 / 3.5, M=1 N=512 K=576 3.2 / 3.1, M=4 N=4608 K=128 4.5 / 3.1.
+  if constexpr (sizeof(TA) == 4) {
+    if (p.M <= kSkinnyM && p.K >= 1024 && split_fits(p) && tiles_of(p, 16) <= 256)
+      return launch_split<W, TO>(p, s);
+  }
   if (p.M <= kSkinnyM && p.a_bytes != 0) {
     const dim3 grid(static_cast<unsigned>((p.N + 15) / 16), static_cast<unsigned>((p.M + 15) / 16));
     if (p.K <= kSkinnyWaves * kSkinnyBatchShort * kBK)
@@ -1497,8 +1557,7 @@ hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
     // tile64, us: M=192 N=576 K=2304 6.6 / 41.4, M=1024 N=512 K=1024 9.5 / 21.5,
     // M=2048 N=512 K=512 (1024 split tiles) 12.7 / 14.2; M=4096 N=512 K=1024
     // (2048) 31.6 / 23.3.
-    const int64_t t32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
-    if (split_fits(p) && t32 <= (p.K >= 512 ? 1024 : 512)) return launch_split<W, TO>(p, s);
+    if (split_fits(p) && tiles_of(p, 32) <= (p.K >= 512 ? 1024 : 512)) return launch_split<W, TO>(p, s);
   }
   if (big >= 256) {
     hipLaunchKernelGGL((tile_kernel<TA, W, TO, 128, 128>), dim3(static_cast<unsigned>(big)),

@@ -2,7 +2,8 @@
 float64 product of the same operands.
 
   split_kernel           fp32 A, few tiles: the eight waves split K (fewer than eight
-                         32-wide chunks, one more than a round, ragged M and N)
+                         32-wide chunks, one more than a round, ragged M and N), 16x16
+                         tiles (up to 256 of them) and 32x32
   dma_tile_kernel        64x64 tiles: 16-bit operands under one 128x128 tile per CU (the
                          bits of the 128x128 tiles), and fp32 operands
   smallk_stream_kernel   K <= 128, whole 128-column tiles: one and several row tiles per
@@ -52,7 +53,8 @@ BF, HF, FL = torch.bfloat16, torch.float16, torch.float32
 
 
 @pytest.mark.parametrize("m,n,k", [(65, 16, 160), (97, 33, 224), (192, 576, 2304), (1000, 130, 288),
-                                   (70, 100, 1024)])
+                                   (70, 100, 1024), (1, 8, 1024), (17, 70, 1312), (64, 1024, 1024),
+                                   (64, 1040, 1056)])
 @pytest.mark.parametrize("wdt,odt", [(BF, FL), (HF, BF), (FL, FL), (FL, BF)])
 def test_waves_split_k(device, m, n, k, wdt, odt):
     run(device, m, n, k, FL, wdt, odt, True)
