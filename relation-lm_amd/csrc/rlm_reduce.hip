@@ -194,8 +194,15 @@ __device__ void fresh_rows(const HiddenParams& p, int64_t t, int64_t r0, int64_t
             const uint32_t o4[4] = {ov[ib][cc][0].x, ov[ib][cc][0].y, ov[ib][cc][0].z, ov[ib][cc][0].w};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-              d += __uint_as_float(w4[k] << 16) * __uint_as_float(o4[k] << 16);
-              d += __uint_as_float(w4[k] & 0xffff0000u) * __uint_as_float(o4[k] & 0xffff0000u);
+              if constexpr (__is_same(T, bf16)) {
+                d += bf16_lo(w4[k]) * bf16_lo(o4[k]);
+                d += bf16_hi(w4[k]) * bf16_hi(o4[k]);
+              } else {
+                typedef T t2 __attribute__((ext_vector_type(2)));
+                const t2 w = __builtin_bit_cast(t2, w4[k]), o = __builtin_bit_cast(t2, o4[k]);
+                d += static_cast<float>(w[0]) * static_cast<float>(o[0]);
+                d += static_cast<float>(w[1]) * static_cast<float>(o[1]);
+              }
             }
           } else {
 #pragma unroll
