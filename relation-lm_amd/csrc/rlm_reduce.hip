@@ -37,7 +37,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRows = 64;   // (query, partner) rows per workgroup
 constexpr int kRC16 = 128;  // relation-dim chunk staged in LDS, 16-bit path
-constexpr int kRC32 = 64;   // relation-dim chunk staged in LDS, fp32 path
+constexpr int kRC32 = 128;  // relation-dim chunk staged in LDS, fp32 path
 constexpr int kPad16 = 8;   // 16-bit elements of row padding (conflict-free b128 reads)
 constexpr int kPad32 = 4;
 
@@ -250,8 +250,8 @@ __host__ __device__ constexpr int fresh_batches() { return kRows; }
 // elements (rows 4*(lane/16)+e of column n), gathered before the matrix-core
 // work so their latency overlaps it.  Row t of the update form is taken from
 // `fresh` instead of the cache row this launch rewrites.
-template <typename T, bool UPDATE>
-__device__ __forceinline__ void gather_bases(const HiddenParams& p, rsrc_t xr, const RowTable& rt,
+template <typename T, bool UPDATE, int NR>
+__device__ __forceinline__ void gather_bases(const HiddenParams& p, rsrc_t xr, const RowTableN<NR>& rt,
                                              int mrow, int n, int c, int64_t t, int64_t b_first,
                                              const float* fresh, int cols, int lane,
                                              float (&xs)[4]) {
@@ -1269,16 +1269,39 @@ __global__ void __launch_bounds__(kMlpThreads) relation_mlp_kernel(const MlpPara
   }
 }
 
-// fp32 / fp16 caches: fp32 products on v_mfma_f32_16x16x4f32.  64 hidden
-// columns per workgroup; waves in 2x2, each 32 x 32.
-template <typename T, bool UPDATE>
+// Four consecutive elements as fp32.
+template <typename T>
+__device__ __forceinline__ float4 buf_load4f(rsrc_t r, uint32_t off) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(float4, buf_load_b128(r, off));
+  } else {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    const t4 v = __builtin_bit_cast(t4, buf_load_b64(r, off));
+    return make_float4(static_cast<float>(v[0]), static_cast<float>(v[1]), static_cast<float>(v[2]),
+                       static_cast<float>(v[3]));
+  }
+}
+
+// fp32 / fp16 caches: fp32 products on v_mfma_f32_16x16x4f32.  A tile of 32 TM
+// rows by 32 TM hidden columns per workgroup; waves in 2x2, each 16 TM x 16 TM.
+// Latency decides at the sizes that fp32 runs at (24 rows x 2304 columns, R = 128:
+// 0.01 GFLOP), so every load of a chunk -- operand rows, W_m rows, expanded-cache
+// halves -- goes out at once in four-element pieces, and an MFMA step reads
+// sixteen k per LDS access: lane group k4 takes k = 16 g + 4 k4 + e for the four
+// steps e (the same k order on both sides).
+// 24 rows x 2304, R = 128, fp32: 17.7 -> 5.2 us; 1024 rows x 1024: 18.0 -> 8.6 us
+// (element loads and element LDS reads of 64 x 64 tiles before).
+template <typename T, bool UPDATE, int TM>
 __global__ void __launch_bounds__(256) hidden_f32_kernel(const HiddenParams p) {
-  constexpr int BN = 64;
+  constexpr int NR = 32 * TM, BN = 32 * TM;
   constexpr int LD = kRC32 + kPad32;
+  constexpr int PR = kRC32 / 4;             // four-element pieces per staged row
+  constexpr int kPieces = NR * PR / 256;    // per thread, of rows and of W_m
   constexpr uint32_t es = sizeof(T);
-  __shared__ float a_s[kRows][LD];
-  __shared__ float w_s[BN][LD];
-  __shared__ RowTable rt;
+  static_assert(!UPDATE || NR == kRows, "the fresh rows go by tiles of kRows");
+  __shared__ __align__(16) float a_s[NR][LD];
+  __shared__ __align__(16) float w_s[BN][LD];
+  __shared__ RowTableN<NR> rt;
   __shared__ float fresh[UPDATE ? fresh_batches() * 2 * BN : 1];
 
   const int tid = threadIdx.x;
@@ -1287,70 +1310,91 @@ __global__ void __launch_bounds__(256) hidden_f32_kernel(const HiddenParams p) {
   // Row tiles of one batch row run on one XCD (one L2 for the rows they gather).
   const int64_t wg = xcd_tile(static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x,
                               static_cast<int64_t>(gridDim.x) * gridDim.y);
-  const int64_t r0 = wg / gridDim.x * kRows;
+  const int64_t r0 = wg / gridDim.x * NR;
   const int n0 = static_cast<int>(wg % gridDim.x) * BN;
   const rsrc_t xr = make_rsrc(p.expanded, p.expanded_bytes);
   const rsrc_t opr = make_rsrc(p.operand, p.operand_bytes);
   const rsrc_t wr_ = make_rsrc(p.wm, p.wm_bytes);
   const rsrc_t outr = make_rsrc(p.out, p.out_bytes);
   const int64_t t_pos = UPDATE ? index_at(p.pos, p.pos_dtype, 0) : -1;  // beside the row loads
-  load_rows<T>(p, r0, rt);
+  float4 vw[kPieces];
+  auto load_w = [&](int rc) {
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+      const int piece = tid + 256 * c;
+      const int n = n0 + piece / PR, r = rc + piece % PR * 4;
+      vw[c] = buf_load4f<T>(wr_, n < p.H && r < p.R
+                                     ? es * (static_cast<uint32_t>(n) * p.R + r) : kNoOffset);
+    }
+  };
+  load_w(0);  // beside the row loads too
+  load_rows<T, NR>(p, r0, rt);
   int64_t b_first;
   const int64_t t = update_setup<T, UPDATE>(p, t_pos, r0, n0, BN, b_first, fresh);
   __syncthreads();
 
-  const int wr = (wave >> 1) * 32;
-  const int wc = (wave & 1) * 32;
+  const int wr = (wave >> 1) * 16 * TM;
+  const int wc = (wave & 1) * 16 * TM;
   const int r16 = lane & 15;
   const int k4 = lane >> 4;
-  float xs[2][2][4];
+  float xs[TM][TM][4];
+  f32x4 acc[TM][TM];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      gather_bases<T, UPDATE>(p, xr, rt, wr + i * 16, n0 + wc + j * 16 + r16, wc + j * 16 + r16,
-                              t, b_first, fresh, BN, lane, xs[i][j]);
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   for (int rc = 0; rc < p.R; rc += kRC32) {
-    if (rc) __syncthreads();
-    for (int idx = tid; idx < kRows * kRC32; idx += 256) {
-      const int row = idx / kRC32;
-      const int r = rc + idx % kRC32;
-      const bool in = r < p.R;
-      const float oa = buf_load_elem<T>(opr, in ? rt.op_a[row] + es * r : kNoOffset);
-      const float op = buf_load_elem<T>(opr, in ? rt.op_p[row] + es * r : kNoOffset);
-      a_s[row][idx % kRC32] = op * oa;
+    float4 va[kPieces], vp[kPieces];
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+      const int piece = tid + 256 * c;
+      const int row = piece / PR, r = rc + piece % PR * 4;
+      va[c] = buf_load4f<T>(opr, r < p.R ? rt.op_a[row] + es * r : kNoOffset);
+      vp[c] = buf_load4f<T>(opr, r < p.R ? rt.op_p[row] + es * r : kNoOffset);
     }
-    for (int idx = tid; idx < BN * kRC32; idx += 256) {
-      const int n = n0 + idx / kRC32;
-      const int r = rc + idx % kRC32;
-      w_s[idx / kRC32][idx % kRC32] = buf_load_elem<T>(
-          wr_, (n < p.H && r < p.R) ? es * (static_cast<uint32_t>(n) * p.R + r) : kNoOffset);
+    if (rc == 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+          gather_bases<T, UPDATE>(p, xr, rt, wr + i * 16, n0 + wc + j * 16 + r16,
+                                  wc + j * 16 + r16, t, b_first, fresh, BN, lane, xs[i][j]);
+    } else {
+      load_w(rc);
+      __syncthreads();  // the chunk before is read
+    }
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+      const int piece = tid + 256 * c;
+      const int row = piece / PR, at = piece % PR * 4;
+      *reinterpret_cast<float4*>(&w_s[row][at]) = vw[c];
+      *reinterpret_cast<float4*>(&a_s[row][at]) = make_float4(
+          vp[c].x * va[c].x, vp[c].y * va[c].y, vp[c].z * va[c].z, vp[c].w * va[c].w);
     }
     __syncthreads();
     const int rlen = p.R - rc < kRC32 ? p.R - rc : kRC32;
-    for (int kk = 0; kk < rlen; kk += 4) {
-      float av[2], bv[2];
+    for (int kk = 0; kk < rlen; kk += 16) {  // (past rlen: staged zeros)
+      f32x4 av[TM], bv[TM];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) av[i] = a_s[wr + i * 16 + r16][kk + k4];
+      for (int i = 0; i < TM; ++i)
+        av[i] = *reinterpret_cast<const f32x4*>(&a_s[wr + i * 16 + r16][kk + 4 * k4]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) bv[j] = w_s[wc + j * 16 + r16][kk + k4];
+      for (int j = 0; j < TM; ++j)
+        bv[j] = *reinterpret_cast<const f32x4*>(&w_s[wc + j * 16 + r16][kk + 4 * k4]);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
     }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TM; ++j)
       store_hidden(p, outr, acc[i][j], xs[i][j], r0, wr + i * 16, n0 + wc + j * 16 + r16, lane);
 }
 
@@ -2254,12 +2298,18 @@ hipError_t launch_hidden(HiddenParams& p, int dtype, bool update, hipStream_t st
     return launch_status("relation_hidden");
   }
   const dim3 grid(static_cast<unsigned>((p.H + 63) / 64), row_tiles);
-#define RLM_HIDDEN_CASE(ID, T)                                                             \
-  if (dtype == ID) {                                                                       \
-    if (update)                                                                            \
-      hipLaunchKernelGGL((hidden_f32_kernel<T, true>), grid, dim3(256), 0, stream, p);     \
-    else                                                                                   \
-      hipLaunchKernelGGL((hidden_f32_kernel<T, false>), grid, dim3(256), 0, stream, p);    \
+  // 32-row, 32-column tiles where 64 x 64 ones leave CUs idle.
+  const dim3 grid32(static_cast<unsigned>((p.H + 31) / 32),
+                    static_cast<unsigned>((p.rows + 31) / 32));
+  const bool small = !update && static_cast<int64_t>(grid.x) * grid.y < 256;
+#define RLM_HIDDEN_CASE(ID, T)                                                                \
+  if (dtype == ID) {                                                                          \
+    if (update)                                                                               \
+      hipLaunchKernelGGL((hidden_f32_kernel<T, true, 2>), grid, dim3(256), 0, stream, p);     \
+    else if (small)                                                                           \
+      hipLaunchKernelGGL((hidden_f32_kernel<T, false, 1>), grid32, dim3(256), 0, stream, p);  \
+    else                                                                                      \
+      hipLaunchKernelGGL((hidden_f32_kernel<T, false, 2>), grid, dim3(256), 0, stream, p);    \
     return launch_status("relation_hidden");                                               \
   }
   RLM_HIDDEN_CASE(RLM_F32, float)

@@ -1,4 +1,5 @@
-"""The relation hidden of fp32 / fp16 caches (hidden_f32_kernel, the update form) against the expression in float64.
+"""The relation hidden of fp32 / fp16 caches (hidden_f32_kernel: 32 x 32 tiles where few
+64 x 64 ones exist, 64 x 64 tiles, the update form) against the expression in float64.
 
 The products op[a] * op[p] are rounded to fp32 once and R of them are summed in fp32: an
 error of (R + 3) x 2^-24 times the sum of the magnitudes at worst; the GELU's slope is at
@@ -8,7 +9,9 @@ import pytest
 import torch
 
 import relation_lm  # noqa: F401
-from relation_lm.kernels.relation_reduce import relation_hidden_cache_update
+from relation_lm.kernels.relation_reduce import (relation_hidden_cache_update,
+                                                 relation_hidden_cached,
+                                                 relation_hidden_cached_seq)
 
 pytestmark = pytest.mark.gpu
 
@@ -37,6 +40,21 @@ def check(got, expanded, operand, a, p, wm):
     assert got.shape == want.shape
     tol = 1.13 * (r + 3) * 2.0 ** -24 * mag + 2e-6
     assert bool(((got.double().cpu() - want).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("b,q,k,h,r", [
+    (1, 1, 1, 1, 8), (4, 1, 6, 2304, 128), (2, 5, 7, 100, 40), (1, 11, 3, 33, 136),
+    (1, 33, 1, 64, 256), (2, 64, 8, 1024, 128), (1, 340, 5, 700, 72)])
+def test_hidden(device, dtype, b, q, k, h, r):
+    args, dev = inputs(device, b, q, k, h, r, 50, dtype)
+    if q == 1:
+        got = relation_hidden_cached(dev[0], dev[1], dev[2][:, 0].contiguous(),
+                                     dev[3][:, 0].contiguous(), dev[4])[:, None]
+    else:
+        got = relation_hidden_cached_seq(*dev)
+    torch.cuda.synchronize()
+    check(got, *args)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
