@@ -515,7 +515,7 @@ __device__ void stage_workgroup(const SelectParams& p, int64_t b, int64_t wbase,
 }
 
 // RING: ring-buffer caches (decode form only, no staged windows).
-// SPLIT: one query per workgroup (decode), its candidate scoring shared by
+// SPLIT: one query per workgroup (decode, few queries), its candidate scoring shared by
 // p.split waves.
 template <typename TA, typename TS, int MODE, bool RING = false, bool SPLIT = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) select_kernel(const SelectParams p) {
@@ -1279,19 +1279,37 @@ hipError_t finish_params(SelectParams& p, const Geometry& g, int64_t local_windo
   return hipSuccess;
 }
 
+// Queries of a sequence up to which each has a workgroup of its own, as in
+// decode: eight to a workgroup leave CUs idle there, and their staging is one
+// more round trip ahead of a chain of them.  Eight / one, us, fp32, by queries x
+// candidates: 128 x 192 24.9 / 14.2, 512 x 192 30.0 / 19.2, 1024 x 192
+// 30.5 / 24.8, 1024 x 384 58.3 / 37.7; 2048 x 192 31.4 / 44.1, 2048 x 384
+// 69.0 / 83.5.
+constexpr int64_t kAloneQueries = 1024;
+
 template <int MODE, bool RING = false>
-hipError_t launch_select(const SelectParams& p, int act_dtype, int stat_dtype,
+hipError_t launch_select(const SelectParams& given, int act_dtype, int stat_dtype,
                          hipStream_t stream) {
-  const int64_t queries = p.B * p.Tq;
+  const int64_t queries = given.B * given.Tq;
   if (queries == 0) return hipSuccess;
+  SelectParams p = given;
+  if (p.W > 1 && queries <= kAloneQueries) {
+    p.W = 1;
+    p.split = std::min(4, (p.CAP + kWave - 1) / kWave);
+    p.tiles = static_cast<int>(p.Tq);
+    p.WR = p.L;
+    p.stage = 0;
+    p.off_wave = 0;
+    p.lds_total = p.split * p.wave_bytes;
+  }
   const dim3 block(p.W * p.split * kWave);
   const dim3 grid(static_cast<unsigned>(p.B * p.tiles));
   const size_t lds = static_cast<size_t>(p.lds_total);
 #define RLM_SELECT_CASE(TA_ID, TA, TS_ID, TS)                                             \
   if (act_dtype == TA_ID && stat_dtype == TS_ID) {                                        \
-    /* ring caches are decode only (one query per workgroup): always the split */        \
-    /* form, which also serves split == 1 */                                              \
-    if (RING || p.split > 1)                                                              \
+    /* one query per workgroup (ring caches are decode only): the split form, */         \
+    /* which also serves split == 1 */                                                    \
+    if (RING || p.W == 1)                                                                 \
       hipLaunchKernelGGL((select_kernel<TA, TS, MODE, RING, true>), grid, block, lds, stream, p); \
     else if constexpr (!RING)                                                             \
       hipLaunchKernelGGL((select_kernel<TA, TS, MODE, RING, false>), grid, block, lds, stream, p); \

@@ -134,3 +134,22 @@ def test_multi_anchor_block_counts(device, context, block, slots):
         want = multi_relation_select_seq(*multi_select_args(upcast(wild), cfg))
         torch.cuda.synchronize()
         check_same(got, want, f"{context}/{block} {value}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(512, 32, 64, 4, 8), (512, 16, 32, 2, 5), (384, 64, 100, 16, 16),
+                                   (448, 32, 1, 2, 3)])
+@pytest.mark.parametrize("strict", [False, True])
+def test_a_workgroup_per_query_gives_the_same_bits(device, dtype, shape, strict):
+    """select_kernel: up to 1024 queries each have a workgroup, beyond eight share one."""
+    context, block, local, top, k = shape
+    cfg = config(context, block, local, top, k, strict, batch=4, seed=5)
+    cast = lambda v: v.to(dtype) if v.dtype == torch.bfloat16 else v
+    dev = {n: cast(v).to(device) for n, v in selection_inputs(cfg).items()}
+    whole = relation_select_packed_seq(*select_args(dev, cfg))
+    shared = {n: v for n, v in dev.items() if v.shape[:1] != (4,) or n.endswith(("gamma", "bias"))}
+    for b in range(4):
+        row = {n: v if n in shared else v[b:b + 1].contiguous() for n, v in dev.items()}
+        got = relation_select_packed_seq(*select_args(row, cfg))
+        torch.cuda.synchronize()
+        check_same(got, [w[b:b + 1] for w in whole], (shape, b))
