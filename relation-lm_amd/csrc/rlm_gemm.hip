@@ -1458,9 +1458,10 @@ template <typename TA, typename W, typename TO>
 hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
   // An fp32 A with long rows: split / skinny, us: M=64 N=576 K=2304 4.9 / 8.4,
   // M=4 N=576 K=2304 4.6 / 6.1, M=32 N=256 K=1024 3.8 / 5.8; M=8 N=1024 K=512
-  // 3.3 / 3.5, M=1 N=512 K=576 3.2 / 3.1, M=4 N=4608 K=128 4.5 / 3.1.
+  // 3.3 / 3.5, M=1 N=512 K=576 3.2 / 3.1, M=4 N=4608 K=128 4.5 / 3.1.  Only the
+  // skinny kernel writes the cache rows of a scatter (nseg).
   if constexpr (sizeof(TA) == 4) {
-    if (p.M <= kSkinnyM && p.K >= 1024 && split_fits(p) && tiles_of(p, 16) <= 256)
+    if (p.nseg == 0 && p.M <= kSkinnyM && p.K >= 1024 && split_fits(p) && tiles_of(p, 16) <= 256)
       return launch_split<W, TO>(p, s);
   }
   if (p.M <= kSkinnyM && p.a_bytes != 0) {

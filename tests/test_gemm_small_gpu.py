@@ -115,3 +115,24 @@ def test_small_k_strided_rows(device):
     torch.cuda.synchronize()
     assert torch.equal(out[:, 256:], ops.relation_linear(a, w, None, BF))
     assert bool((out[:, :256] == 0).all())
+
+
+@pytest.mark.parametrize("m,k", [(1, 1024), (24, 1056), (64, 2304), (24, 992)])
+@pytest.mark.parametrize("wdt", [BF, HF])
+def test_long_rows_reach_the_caches(device, m, k, wdt):
+    """fp32 rows against a 16-bit weight, at lengths where the product alone is split: the
+    cache-row scatter still writes the caches."""
+    g = torch.Generator().manual_seed(m + k)
+    a = torch.randn(m, k, generator=g).to(device)
+    w = (torch.randn(96, k, generator=g) / np.sqrt(k)).to(wdt).to(device)
+    caches = [torch.zeros(m, 8, n, device=device) for n in (16, 16, 32, 32)]
+    out = ops.packed_projection_to_caches(a, w, *caches, torch.tensor(5, device=device), False)
+    torch.cuda.synchronize()
+    lo = 0
+    for c in caches:
+        n = c.size(2)
+        assert torch.equal(c[:, 5], out[:, lo:lo + n]) and bool(c[:, 5].any())
+        assert not bool(c[:, [0, 1, 2, 3, 4, 6, 7]].any())
+        lo += n
+    a64, w64 = a.to(wdt).double(), w.double()
+    assert bool(((out.double() - a64 @ w64.T).abs() <= 1e-5 * (a64.abs() @ w64.abs().T) + 1e-6).all())
