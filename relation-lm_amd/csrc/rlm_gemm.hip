@@ -1475,8 +1475,11 @@ hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
     return launch_status("linear");
   }
   const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128);
+  // The small-K kernels load a whole row of K columns whatever K is; an empty
+  // reduction (out = bias) goes to the kernels that loop over K.
+  const bool small_k = p.K > 0 && p.K <= 128 && p.K % 32 == 0 && p.a_bytes != 0;
   if constexpr (__is_same(TA, W)) {
-    if (p.K <= 128 && p.K % 32 == 0 && p.a_bytes != 0 && p.N % 128 == 0 &&
+    if (small_k && p.N % 128 == 0 &&
         (p.ldo * static_cast<int64_t>(sizeof(TO))) % 16 == 0 &&
         (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0) {
       switch (p.K / 32) {
@@ -1487,7 +1490,7 @@ hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
       }
     }
   }
-  if (p.K <= 128 && p.K % 32 == 0 && p.a_bytes != 0) {
+  if (small_k) {
     const dim3 grid(static_cast<unsigned>(big));
     switch (p.K / 32) {
       case 1: {

@@ -136,3 +136,16 @@ def test_long_rows_reach_the_caches(device, m, k, wdt):
         lo += n
     a64, w64 = a.to(wdt).double(), w.double()
     assert bool(((out.double() - a64 @ w64.T).abs() <= 1e-5 * (a64.abs() @ w64.abs().T) + 1e-6).all())
+
+
+@pytest.mark.parametrize("adt,wdt,odt", [(BF, BF, BF), (HF, HF, FL), (FL, BF, FL), (FL, FL, FL)])
+@pytest.mark.parametrize("m,n", [(5, 128), (100, 256), (4100, 1024), (130, 72)])
+def test_empty_reduction_is_the_bias(device, m, n, adt, wdt, odt):
+    """K = 0 reads neither operand (their pointers are null here): every output row is the bias."""
+    x = torch.empty(m, 8, dtype=adt, device=device)[:, :0]
+    w = torch.empty(n, 0, dtype=wdt, device=device).as_strided((n, 0), (0, 1))
+    b = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(wdt).to(device)
+    out = torch.full((m, n), float("nan"), dtype=odt, device=device)
+    ops.relation_linear_out(x, w, b, out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, b.to(odt).expand(m, n))
