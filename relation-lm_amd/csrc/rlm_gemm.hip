@@ -1547,13 +1547,20 @@ hipError_t launch_typed(const GemmParams& p, hipStream_t s) {
   }
   if (dma_fits<TA, W, TO>(p)) {
     // 256x256 tiles (eight waves of 128x64) once they fill the chip; 128x128
-    // (four waves, two workgroups per CU) below that; 64x64 where even those are
-    // fewer than the CUs.  The k order is the same, so are the bits.  128 vs 64:
-    // M=3584 N=512 K=576 (112 tiles) 8.7 / 6.9 us, M=4096 N=768 K=3072 (192)
-    // 35.7 / 31.7, M=8192 N=512 K=576 (256) 10.6 / 12.1.
+    // (four waves, two workgroups per CU) below that; 64x64 where those are at
+    // most three per CU, the workgroups that run at once (a fourth starts another
+    // round).  The k order is the same, so are the bits.  128 / 64, us:
+    //   M=3584 N=512 K=576 (448 tiles of 64)    8.6 / 6.8    M=3072 N=768 K=576 (576)   9.0 / 8.8
+    //   M=4096 N=768 K=3072 (768)              35.7 / 31.7   M=3072 N=1024 K=1536 (768) 19.1 / 16.5
+    //   M=3200 N=1024 K=576 (800)               9.7 / 11.1   M=3584 N=1024 K=3072 (896) 36.2 / 40.5
+    // One column of 128x128 tiles (N <= 128) with a longer K pays up to four per CU:
+    //   M=28672 N=128 (896) K=192 7.0 / 7.3, K=768 15.8 / 14.9, K=2304 35.8 / 33.4
+    // and from one 128x128 tile per CU on it no longer does:
+    //   M=65000 N=64 (1016 of 64, 508 of 128) K=2304 56.6 / 62.8
     if (((p.M + 255) / 256) * ((p.N + 255) / 256) >= 256)
       return launch_dma<W, TO, 256, 256, 2, 4, 2, kDmaSliceK>(p, s);
-    if (big >= 256) return launch_dma<W, TO, 128, 128, 2, 2, 2, kDmaSliceK>(p, s);
+    if (big >= 256 || tiles_of(p, 64) > (p.N <= 128 && p.K >= 512 ? 1024 : 768))
+      return launch_dma<W, TO, 128, 128, 2, 2, 2, kDmaSliceK>(p, s);
     return launch_dma<W, TO, 64, 64, 2, 2, 2, kDmaSliceK>(p, s);
   }
   if constexpr (sizeof(TA) == 4) {
