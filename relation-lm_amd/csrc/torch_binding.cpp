@@ -818,15 +818,24 @@ std::tuple<at::Tensor, at::Tensor> relation_hidden_linear_norm_reduce_output(
 // Whether the relation MLP kernel with the norm-reduce as its epilogue (64-row
 // tiles, plus a launch that packs the weights) is the faster form of the relation
 // reduce.
-//   Against the fused kernel (128-row tiles, K padded to a power of two): one tile
-//   per CU at a time, a 64-row round about 0.6 of a 128-row one.  D=512: B=8 T=512
-//   K=8 H=512 (2 rounds / 1) 43.8 / 34.3 us, B=8 T=2048 H=1024 (8 / 4) 261 / 256;
-//   B=4 T=256 K=8 D=256 H=1024 (1 / 1) 29.6 / 43.5, B=5 T=1728 K=5 D=384 H=512
-//   (3 / 3) 62 / 91.
+//   Against the fused kernel (128-row tiles, K padded to a power of two), by rounds
+//   of one tile per CU: a 64-row round takes 0.56 of a 128-row one and a share that
+//   falls with the hidden dim (the epilogue, the packing), more at few columns or
+//   many partners, less at d_model 384 (the fused kernel's waves are uneven there).
+//   The form of second_weight does not enter, so that both forms give the same bits.
+//   Fused / MLP, us, by rounds of 64 / 128 rows:
+//     D=128 R=64    K=5 H=128 (3 / 2) 20.1 / 26.2, K=1 H=128 (1 / 1) 9.7 / 10.4
+//   MLP as a share of the fused time:
+//     D=128 R=64    H=1024 (1 / 1) 0.61-0.67, (3 / 2) 0.82-0.86, (2 / 1) 1.09-1.12
+//     D=384 R=128   H=512 (2 / 1) 0.94-0.99, (3 / 2) 0.73; H=128 (2 / 1) 1.41
+//     D=512 R=128   H=256 (1 / 1) 0.71-0.91, (3 / 2) 1.04-1.14; H=512 (3 / 2) 0.93-1.02
+//   Over 2546 shapes it is at most 7% above the fused time and 0.6% above the better
+//   of the two on average.
 //   Against the three ops (other d_model): its tiles' chunk loop is a chain of
 //   H / 128 steps however few tiles there are.  H=2304 D=576: 768 rows 57 / 27 us,
 //   1024 58 / 37, 2048 58 / 82, 28672 134 / 386; H=512 D=320: 512 rows 18.6 / 17.4.
-bool mlp_reduce_faster(const at::Tensor& partner_index, bool fused_fits) {
+bool mlp_reduce_faster(const at::Tensor& partner_index, int64_t hidden_dim, int64_t d_model,
+                       bool fused_fits) {
   const int64_t queries = partner_index.size(0) * partner_index.size(1);
   const int64_t K = partner_index.size(2);
   if (K < 1 || K > 16) return false;
@@ -835,7 +844,9 @@ bool mlp_reduce_faster(const at::Tensor& partner_index, bool fused_fits) {
   while (padded < K) padded *= 2;
   const int64_t rounds64 = (queries + (64 / K) * 256 - 1) / ((64 / K) * 256);
   const int64_t rounds128 = (queries * padded + 128 * 256 - 1) / (128 * 256);
-  return 5 * rounds128 > 3 * rounds64;
+  double round = 0.56 + (d_model <= 256 || K > 8 ? 64.0 : 48.0) / static_cast<double>(hidden_dim);
+  if (d_model == 384) round *= 0.9;
+  return static_cast<double>(rounds128) > round * static_cast<double>(rounds64);
 }
 
 at::Tensor relation_reduce_fused_seq(const at::Tensor& expanded_cache,
@@ -868,7 +879,8 @@ at::Tensor relation_reduce_fused_seq(const at::Tensor& expanded_cache,
     TORCH_CHECK(fits || !frag, op, ": a second_weight in fragment order needs the fused kernel's "
                 "shapes (bf16, d_model 128/256/384/512, K <= 16, relation dim 32/64/128); "
                 "pass the [D,H] weight for other shapes");
-    if (mlp_reduce_faster(partner_index, fits) &&
+    const int64_t hidden_dim = product_weight.dim() == 2 ? product_weight.size(0) : 0;
+    if (mlp_reduce_faster(partner_index, hidden_dim, d_model, fits) &&
         rlm_relation_mlp_reduce_seq_fits(&e, &o, &pi, &wm, &w2)) {
       at::Tensor out = at::empty({partner_index.size(0), partner_index.size(1), d_model},
                                  f32(operand_cache));

@@ -5,25 +5,14 @@ from __future__ import annotations
 
 import pytest
 import torch
-from torch.profiler import ProfilerActivity, profile
+from launched import launched
 
 from relation_lm import _native  # noqa: F401  (registers torch.ops.relation_lm)
+from relation_lm.kernels.relation_reduce import mfma_fragments, relation_reduce_fused_seq
 
 pytestmark = pytest.mark.gpu
 ops = torch.ops.relation_lm
 BF, FL = torch.bfloat16, torch.float32
-
-
-def launched(call):
-    """Names of the kernels one call launches."""
-    call()
-    torch.cuda.synchronize()
-    with profile(activities=[ProfilerActivity.CUDA]) as prof:
-        call()
-        torch.cuda.synchronize()
-    names = [e.key for e in prof.key_averages() if "rlm::" in e.key]
-    assert names
-    return " ".join(names)
 
 
 @pytest.mark.parametrize("m,n,k,tile", [
@@ -36,3 +25,32 @@ def test_linear_tile_size(device, m, n, k, tile):
     a, w = torch.ones(m, k, dtype=BF, device=device), torch.ones(n, k, dtype=BF, device=device)
     names = launched(lambda: ops.relation_linear(a, w, None, BF))
     assert "dma_tile_kernel" in names and f"{tile}, {tile}," in names, names
+
+
+FUSED, MLP, CHAIN = "fused_reduce_kernel", "relation_mlp_kernel", "norm_reduce"
+
+
+@pytest.mark.parametrize("queries,k,d,h,r,frag,kernel", [
+    (4096, 8, 512, 512, 128, True, FUSED),     # two 64-row rounds against one of 128 rows
+    (3840, 5, 128, 128, 64, False, FUSED),     # 2 / 1, few columns
+    (8192, 5, 128, 128, 64, True, FUSED),      # 3 / 2
+    (200, 8, 128, 128, 128, False, FUSED),     # 1 / 1, one hidden chunk
+    (4000, 12, 256, 256, 128, False, FUSED),   # 4 / 2
+    (200, 8, 512, 128, 128, False, MLP), (200, 5, 128, 512, 64, False, MLP),
+    (200, 5, 128, 512, 64, True, MLP),         # the weight's order does not choose
+    (5000, 6, 512, 1024, 128, False, MLP),     # 2 / 2
+    (200, 8, 576, 256, 128, False, MLP), (191, 8, 576, 256, 128, False, CHAIN)])
+def test_relation_reduce_kernel(device, queries, k, d, h, r, frag, kernel):
+    g = torch.Generator().manual_seed(queries + d)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g).to(BF).to(device)
+
+    wm, w2 = rand(h, r), rand(d, h)
+    anchor = torch.zeros(1, queries, dtype=torch.int32, device=device)
+    partner = torch.zeros(1, queries, k, dtype=torch.int32, device=device)
+    names = launched(lambda: relation_reduce_fused_seq(
+        rand(1, 64, 2 * h), rand(1, 64, r), anchor, partner, wm, mfma_fragments(w2) if frag else w2,
+        rand(d), torch.zeros(1, queries, k, device=device), rand(d), rand(d),
+        torch.arange(queries, device=device), 1e-5))
+    assert kernel in names and not any(x in names for x in {FUSED, MLP, CHAIN} - {kernel}), names
