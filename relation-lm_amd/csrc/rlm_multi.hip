@@ -285,14 +285,16 @@ struct BlockStatsParams {
 // One thread per (batch row, block, channel); consecutive threads take
 // consecutive channels, so every key row is read coalesced.  Mean, then the mean
 // squared deviation, fp32, rows in order.  Latency bounds it (B=4, T=4096, block
-// 64, 64 channels: 2 MB, 16384 threads): a thread has 64 rows in flight and keeps
-// them for the second sum, and 64-thread workgroups reach every CU: 5.4 us, where
-// a load per add and 64 workgroups of 256 took 29.
-constexpr int kStatRows = 64;   // rows held by a thread
-constexpr int kStatThreads = 64;
-
-template <typename T>
-__global__ void __launch_bounds__(kStatThreads) block_stats_kernel(const BlockStatsParams p) {
+// 64, 64 channels: 2 MB, 16384 threads): a thread has ROWS rows in flight and keeps
+// them for the second sum, and 64-thread workgroups reach every CU: 4.2 us, where
+// a load per add and workgroups of 256 took 14.2.  ROWS is the block's length up to
+// 1, 2, 8, 16, 32 or 64 (longer blocks run in pieces of 64): rows past the block are
+// loaded again and dropped, and with 64 of them for every length short blocks took
+// longer than with a load per add.  A load per add / always 64 / this, us: B=8 T=512
+// block 4, 128 channels 3.1 / 5.5 / 3.1; B=32 T=4096 block 16 7.3 / 13.2 / 6.5; B=8 T=4096
+// block 2 6.4 / - / 6.2 (8 rows and 64 threads: 8.3); B=16 T=4096 block 32 8.4 / - / 4.2.
+template <typename T, int ROWS, int THREADS>
+__global__ void __launch_bounds__(THREADS) block_stats_kernel(const BlockStatsParams p) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t total = p.B * p.NB * p.C;
   if (i >= total) return;
@@ -301,30 +303,49 @@ __global__ void __launch_bounds__(kStatThreads) block_stats_kernel(const BlockSt
   const int j = static_cast<int>(bj % p.NB);
   const int64_t b = bj / p.NB;
   const T* k = static_cast<const T*>(p.keys) + (b * p.T + static_cast<int64_t>(j) * p.BS) * p.C + c;
-  T v[kStatRows];
+  T v[ROWS];
   auto load = [&](int r0) {
 #pragma unroll
-    for (int u = 0; u < kStatRows; ++u)
+    for (int u = 0; u < ROWS; ++u)
       v[u] = k[static_cast<int64_t>(min(r0 + u, p.BS - 1)) * p.C];
   };
   float sum = 0.0f;
-  for (int r0 = 0; r0 < p.BS; r0 += kStatRows) {
+  for (int r0 = 0; r0 < p.BS; r0 += ROWS) {
     load(r0);
 #pragma unroll
-    for (int u = 0; u < kStatRows; ++u) sum = r0 + u < p.BS ? sum + to_f32(v[u]) : sum;
+    for (int u = 0; u < ROWS; ++u) sum = r0 + u < p.BS ? sum + to_f32(v[u]) : sum;
   }
   const float mean = sum / static_cast<float>(p.BS);
   float sq = 0.0f;
-  for (int r0 = 0; r0 < p.BS; r0 += kStatRows) {
-    if (p.BS > kStatRows) load(r0);
+  for (int r0 = 0; r0 < p.BS; r0 += ROWS) {
+    if (p.BS > ROWS) load(r0);
 #pragma unroll
-    for (int u = 0; u < kStatRows; ++u) {
+    for (int u = 0; u < ROWS; ++u) {
       const float d = to_f32(v[u]) - mean;
       sq = r0 + u < p.BS ? fmaf(d, d, sq) : sq;
     }
   }
   p.mean[i] = mean;
   p.std[i] = sqrtf(sq / static_cast<float>(p.BS));
+}
+
+template <typename T, int ROWS, int THREADS = 64>
+hipError_t launch_block_stats(const BlockStatsParams& p, hipStream_t stream) {
+  const int64_t total = p.B * p.NB * p.C;
+  hipLaunchKernelGGL((block_stats_kernel<T, ROWS, THREADS>),
+                     dim3(static_cast<unsigned>((total + THREADS - 1) / THREADS)), dim3(THREADS), 0,
+                     stream, p);
+  return launch_status("block_statistics");
+}
+
+template <typename T>
+hipError_t launch_block_stats(const BlockStatsParams& p, hipStream_t stream) {
+  if (p.BS == 1) return launch_block_stats<T, 1, 256>(p, stream);
+  if (p.BS == 2) return launch_block_stats<T, 2, 256>(p, stream);
+  if (p.BS <= 8) return launch_block_stats<T, 8>(p, stream);
+  if (p.BS <= 16) return launch_block_stats<T, 16>(p, stream);
+  if (p.BS <= 32) return launch_block_stats<T, 32>(p, stream);
+  return launch_block_stats<T, 64>(p, stream);
 }
 
 template <int G>
@@ -550,19 +571,8 @@ extern "C" hipError_t rlm_block_statistics(const rlm_tensor* keys, int64_t block
   p.keys = keys->data;
   p.mean = static_cast<float*>(out_mean->data);
   p.std = static_cast<float*>(out_std->data);
-  const int64_t total = B * NB * C;
-  if (total == 0) return hipSuccess;
-  const dim3 grid(static_cast<unsigned>((total + kStatThreads - 1) / kStatThreads));
-  switch (keys->dtype) {
-    case RLM_F32:
-      hipLaunchKernelGGL((block_stats_kernel<float>), grid, dim3(kStatThreads), 0, stream, p);
-      break;
-    case RLM_BF16:
-      hipLaunchKernelGGL((block_stats_kernel<bf16>), grid, dim3(kStatThreads), 0, stream, p);
-      break;
-    default:
-      hipLaunchKernelGGL((block_stats_kernel<f16>), grid, dim3(kStatThreads), 0, stream, p);
-      break;
-  }
-  return launch_status("block_statistics");
+  if (B * NB * C == 0) return hipSuccess;
+  if (keys->dtype == RLM_F32) return launch_block_stats<float>(p, stream);
+  if (keys->dtype == RLM_BF16) return launch_block_stats<bf16>(p, stream);
+  return launch_block_stats<f16>(p, stream);
 }

@@ -54,3 +54,25 @@ def test_relation_reduce_kernel(device, queries, k, d, h, r, frag, kernel):
         rand(d), torch.zeros(1, queries, k, device=device), rand(d), rand(d),
         torch.arange(queries, device=device), 1e-5))
     assert kernel in names and not any(x in names for x in {FUSED, MLP, CHAIN} - {kernel}), names
+
+
+@pytest.mark.parametrize("block,rows", [(1, 1), (2, 2), (3, 8), (8, 8), (9, 16), (16, 16), (17, 32),
+                                        (32, 32), (33, 64), (64, 64), (200, 64)])
+@pytest.mark.parametrize("dtype", [FL, BF])
+def test_block_statistics_rows(device, block, rows, dtype):
+    """A thread holds the block's rows up to the next instance, no more; the statistics are fp32
+    sums in row order: n + 2 roundings of 2^-24 of sum |x| and of sum d^2 (the mean's own error
+    enters the deviation's square root once)."""
+    x = torch.randn(3, 4 * block, 40, generator=torch.Generator().manual_seed(block)).to(dtype)
+    keys = x.to(device)
+    names = launched(lambda: ops.block_statistics(keys, block))
+    assert f", {rows}, " in names, names
+    mean, std = ops.block_statistics(keys, block)
+    torch.cuda.synchronize()
+    x64 = x.double().view(3, 4, block, 40)
+    want = x64.mean(2)
+    dev = (x64 - want[:, :, None]).square().mean(2).sqrt()
+    eps = (block + 2) * 2.0 ** -24
+    tol = eps * x64.abs().mean(2)
+    assert bool(((mean.double().cpu() - want).abs() <= tol).all())
+    assert bool(((std.double().cpu() - dev).abs() <= eps * dev + tol).all())
