@@ -410,7 +410,7 @@ __device__ __forceinline__ int emit(const MultiTileParams& p, const MRec& R, int
 // else k = K, ties to the lowest candidate lane.  The record's anchors so far
 // (taken[0..nact)) are not candidates.  `qrow` is the float64 query and `qn1` its L1 norm.  Returns the
 // anchor position (ANCHOR; -1 for none).
-template <bool ANCHOR, bool SINGLE, bool ANY>
+template <bool ANCHOR, bool SINGLE>
 __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int lane,
                             const double* qrow, float qn1, float kmax, rsrc_t keys, int64_t b,
                             int s, int64_t orow) {
@@ -420,10 +420,10 @@ __device__ int exact_select(const MultiTileParams& p, const MLds& L, int qi, int
   float* sc = L.sc + qi * (p.q_bytes >> 2);
   const float eps = kErrScale * qn1 * kmax;
   // Scores that may not be finite (wave-uniform): the filter's bound does not
-  // hold, so every candidate becomes a member (ANY only).
-  constexpr bool kRaw = ANY && (SINGLE || !ANCHOR);
-  const bool wild = ANY && !(eps <= kErrFinite);
-  if (wild) {
+  // hold, so every candidate becomes a member.
+  constexpr bool kRaw = SINGLE || !ANCHOR;
+  const bool wild = __builtin_amdgcn_readfirstlane(eps <= kErrFinite ? 0 : 1) != 0;
+  if (__builtin_expect(wild, 0)) {
     for (int c = lane; c < p.CAP; c += kWave) {
       bool v;
       cand_pos(p, R, c, t, ls, v);
@@ -724,10 +724,8 @@ __device__ __forceinline__ float routing_kmax(const MLds& L) {
 // SINGLE: the single-anchor selection (S = 1) with select_kernel's results: slot
 // 0 is active at every position, a query without a candidate reports position
 // t - L + 1 and still routes its partners, from its query-side row alone.
-// ANY: scores that may not be finite get the per-query kernels' results (the
-// multi-anchor instance for NB % 4 == 0 keeps the filtered results for those,
-// and 1.5% of its time).
-template <typename TS, bool SINGLE, bool ANY>
+// Scores that may not be finite get the per-query kernels' results in either form.
+template <typename TS, bool SINGLE>
 __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTileParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const MLds L = carve(p, smem);
@@ -822,7 +820,7 @@ __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTilePa
         }
         continue;
       }
-      const int anchor = exact_select<true, SINGLE, ANY>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax,
+      const int anchor = exact_select<true, SINGLE>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax,
                                             akeys, b, s, orow);
       if (anchor >= 0 && lane == 0) {
         MRec& R = L.qr[qi];
@@ -893,7 +891,7 @@ __global__ void __launch_bounds__(kMThreads) multi_tile_kernel(const MultiTilePa
       const int64_t qrow = query_row(qi, active);
       const int64_t orow = qrow * p.S + s;
       if (L.qr[qi].on) {
-        exact_select<false, SINGLE, ANY>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax, pkeys, b, s,
+        exact_select<false, SINGLE>(p, L, qi, lane, L.eq + qi * kMQRow, l1_norm(qi), kmax, pkeys, b, s,
                             orow);
       } else if (active) {  // inactive (or anchorless) slot: every entry exhausted
         for (int k = lane; k < p.K; k += kWave) {
@@ -938,26 +936,23 @@ hipError_t multi_tile_launch(const MultiTileParams& p, int stat_dtype, hipStream
   const dim3 block(kMThreads);
   const dim3 grid(static_cast<unsigned>(p.B * p.tiles));
   const size_t lds = static_cast<size_t>(p.lds_total);
-  const bool any = p.single || (p.NB & 3) != 0;
-#define RLM_MTILE_CASE(TS_ID, TS, SINGLE, ANY)                                             \
-  if (stat_dtype == TS_ID && p.single == SINGLE && any == ANY) {                                         \
+#define RLM_MTILE_CASE(TS_ID, TS, SINGLE)                                                  \
+  if (stat_dtype == TS_ID && p.single == SINGLE) {                                         \
     static const hipError_t attr = hipFuncSetAttribute(                                    \
-        reinterpret_cast<const void*>(&multi_tile_kernel<TS, SINGLE, ANY>),                     \
+        reinterpret_cast<const void*>(&multi_tile_kernel<TS, SINGLE>),                     \
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                           \
     if (attr != hipSuccess) {                                                              \
       set_error("relation selection (tile): cannot reserve LDS: %s",                       \
                 hipGetErrorString(attr));                                                  \
       return attr;                                                                         \
     }                                                                                      \
-    hipLaunchKernelGGL((multi_tile_kernel<TS, SINGLE, ANY>), grid, block, lds, stream, p);      \
+    hipLaunchKernelGGL((multi_tile_kernel<TS, SINGLE>), grid, block, lds, stream, p);      \
     return launch_status("relation selection (tile)");                                     \
   }
-  RLM_MTILE_CASE(RLM_F32, float, false, false)
-  RLM_MTILE_CASE(RLM_BF16, bf16, false, false)
-  RLM_MTILE_CASE(RLM_F32, float, false, true)
-  RLM_MTILE_CASE(RLM_BF16, bf16, false, true)
-  RLM_MTILE_CASE(RLM_F32, float, true, true)
-  RLM_MTILE_CASE(RLM_BF16, bf16, true, true)
+  RLM_MTILE_CASE(RLM_F32, float, false)
+  RLM_MTILE_CASE(RLM_BF16, bf16, false)
+  RLM_MTILE_CASE(RLM_F32, float, true)
+  RLM_MTILE_CASE(RLM_BF16, bf16, true)
 #undef RLM_MTILE_CASE
   set_error("relation selection (tile): unsupported statistics dtype %s",
             dtype_name(stat_dtype));

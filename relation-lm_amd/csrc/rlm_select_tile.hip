@@ -305,7 +305,7 @@ __device__ void head_scores(const TileParams& p, const Lds& L, int side, int wav
 // Keys per query in `blk`: even, so that a row's keys are read two at a time.
 __host__ __device__ __forceinline__ int blk_stride(const TileParams& p) { return (p.NB + 1) & ~1; }
 
-template <int HL, bool ANY>
+template <int HL>
 __device__ __forceinline__ void block_keys(const TileParams& p, const Lds& L, int g) {
   constexpr int H = 1 << HL;
   const int q = g / p.NB;
@@ -328,16 +328,15 @@ __device__ __forceinline__ void block_keys(const TileParams& p, const Lds& L, in
   const int ls = t - p.L + 1 > 0 ? t - p.L + 1 : 0;
   const int end = (j + 1) * p.BS - 1;
   const bool eligible = end <= t && (!p.strict || end < ls);
-  uint64_t* row = L.blk + q * (ANY ? blk_stride(p) : p.NB);
+  uint64_t* row = L.blk + q * blk_stride(p);
   row[j] = select_key(eligible ? static_cast<float>(lse) : -INFINITY, static_cast<uint32_t>(j));
-  if (ANY && j == p.NB - 1 && (p.NB & 1)) row[p.NB] = 0;  // the pad: below every key
+  if (j == p.NB - 1 && (p.NB & 1)) row[p.NB] = 0;  // the pad: below every key
 }
 
-template <bool ANY>
 __device__ __forceinline__ void block_ranks(const TileParams& p, const Lds& L, int g) {
   const int q = g / p.NB;
   const int j = g - q * p.NB;
-  const uint64_t* row = L.blk + q * (ANY ? blk_stride(p) : p.NB);
+  const uint64_t* row = L.blk + q * blk_stride(p);
   const uint64_t kj = row[j];
   int rank = 0;
   for (int k = 0; k < p.NB; k += 2) {
@@ -355,16 +354,15 @@ __device__ __forceinline__ void block_ranks(const TileParams& p, const Lds& L, i
 
 // The picks phase of one stream, between two workgroup barriers: keys, then
 // (once every key of a query is written) ranks.
-template <bool ANY>
 __device__ __forceinline__ void block_picks(const TileParams& p, const Lds& L, int wave, int lane) {
   const int g = wave * kWave + lane;
   const bool mine = g < kQ * p.NB;
   if (mine) {
     switch (p.H_log2) {
-      case 0: block_keys<0, ANY>(p, L, g); break;
-      case 1: block_keys<1, ANY>(p, L, g); break;
-      case 2: block_keys<2, ANY>(p, L, g); break;
-      default: block_keys<3, ANY>(p, L, g); break;
+      case 0: block_keys<0>(p, L, g); break;
+      case 1: block_keys<1>(p, L, g); break;
+      case 2: block_keys<2>(p, L, g); break;
+      default: block_keys<3>(p, L, g); break;
     }
   }
   // A query's keys sit in one wave when NB divides 64, else they may span two.
@@ -373,7 +371,7 @@ __device__ __forceinline__ void block_picks(const TileParams& p, const Lds& L, i
   } else {
     wave_sync();
   }
-  if (mine) block_ranks<ANY>(p, L, g);
+  if (mine) block_ranks(p, L, g);
 }
 
 // Clears the wave's query's candidate table: the local window (positions
@@ -474,7 +472,7 @@ __device__ __forceinline__ int emit(const TileParams& p, const QRec& R, int64_t 
 // query qi, written to the outputs.  ANCHOR: k = 1, ties to the lowest position
 // (returns the anchor); else k = p.K, ties to the lowest candidate lane, and
 // `exclude` is not a candidate.  `qrow` is the float64 query, `qn1` its L1 norm.
-template <bool ANCHOR, bool ANY>
+template <bool ANCHOR>
 __device__ int exact_select(const TileParams& p, const Lds& L, int qi, int lane, int t, int ls,
                             int exclude, const double* qrow, float qn1, float kmax, bool active,
                             int64_t qrow_out) {
@@ -531,13 +529,19 @@ __device__ int exact_select(const TileParams& p, const Lds& L, int qi, int lane,
   const float eps = kErrScale * qn1 * kmax;
   // Scores that may not be finite (wave-uniform): the filter's bound does not
   // hold, so every candidate becomes a member, and the list is what
-  // select_kernel gives for such scores (ANY only).
-  const bool wild = ANY && !(eps <= kErrFinite);
-  const float thr = theta - (2.0f * eps + kErrAbs);
+  // select_kernel gives for such scores.  A scalar branch: as a lane condition
+  // it became selects on every candidate (B=8, T=512: 17.5 / 18.0 us).
+  const bool wild = __builtin_amdgcn_readfirstlane(eps <= kErrFinite ? 0 : 1) != 0;
+  float thr = theta - (2.0f * eps + kErrAbs);
+  if (__builtin_expect(wild, 0)) {
+    thr = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kMaxNCL; ++i) st[i] = ok[i] ? 0.0f : -INFINITY;
+  }
   uint32_t mask = 0;
 #pragma unroll
   for (int i = 0; i < kMaxNCL; ++i)
-    if (wild ? ok[i] : st[i] > -INFINITY && st[i] >= thr) mask |= 1u << i;
+    if (st[i] > -INFINITY && st[i] >= thr) mask |= 1u << i;
   int mi[kMaxNCL];
   const int members = number_members<kMaxNCL>(mask, mi);
   uint64_t* list = L.list + qi * kListCap;
@@ -777,10 +781,7 @@ __device__ void expand_rest(const TileParams& p, unsigned char* stage, int64_t w
 }
 
 // XP: the launch also projects the expanded cache (TileParams::x_*).
-// ANY: any number of blocks up to 64, and for scores that may not be finite the
-// per-query kernel's results (the instance for NB % 4 == 0 keeps the filtered
-// results for those, and 1% of its time).
-template <typename TS, bool XP, bool ANY>
+template <typename TS, bool XP>
 __global__ void __launch_bounds__(kThreads) select_tile_kernel(const TileParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Lds L = carve(p, smem);
@@ -881,9 +882,9 @@ __global__ void __launch_bounds__(kThreads) select_tile_kernel(const TileParams 
   }
   __syncthreads();  // B1: s~ and the head scores complete
 
-  block_picks<ANY>(p, L, wave, lane);
+  block_picks(p, L, wave, lane);
   __syncthreads();  // every query's picks are in its candidate table
-  const int anchor = exact_select<true, ANY>(p, L, qi, lane, t, ls, -1, L.eq + qi * kQRow, qn1, kmax,
+  const int anchor = exact_select<true>(p, L, qi, lane, t, ls, -1, L.eq + qi * kQRow, qn1, kmax,
                                         active, qrow);
   clear_table(p, L, qi, lane, t);
 
@@ -950,9 +951,9 @@ __global__ void __launch_bounds__(kThreads) select_tile_kernel(const TileParams 
   }
   __syncthreads();  // B4: s~ and the head scores complete
 
-  block_picks<ANY>(p, L, wave, lane);
+  block_picks(p, L, wave, lane);
   __syncthreads();  // every query's picks are in its candidate table
-  exact_select<false, ANY>(p, L, qi, lane, t, ls, anchor, L.eq + qi * kQRow, qn1, kmax, active, qrow);
+  exact_select<false>(p, L, qi, lane, t, ls, anchor, L.eq + qi * kQRow, qn1, kmax, active, qrow);
 }
 
 }  // namespace
@@ -989,26 +990,22 @@ hipError_t select_tile_launch(const TileParams& p, int stat_dtype, hipStream_t s
   const size_t lds = static_cast<size_t>(p.lds_total);
   // The LDS opt-in above 64 KiB is a per-process function attribute (set once
   // per instantiation, for the full 160 KiB).
-#define RLM_TILE_CASE(TS_ID, TS, XP, ANY)                                                 \
-  if (stat_dtype == TS_ID && (p.x_out != nullptr) == XP && ((p.NB & 3) != 0) == ANY) {                                \
+#define RLM_TILE_CASE(TS_ID, TS, XP)                                                      \
+  if (stat_dtype == TS_ID && (p.x_out != nullptr) == XP) {                                \
     static const hipError_t attr = hipFuncSetAttribute(                                   \
-        reinterpret_cast<const void*>(&select_tile_kernel<TS, XP, ANY>),                       \
+        reinterpret_cast<const void*>(&select_tile_kernel<TS, XP>),                       \
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                          \
     if (attr != hipSuccess) {                                                             \
       set_error("relation_select (tile): cannot reserve LDS: %s", hipGetErrorString(attr)); \
       return attr;                                                                        \
     }                                                                                     \
-    hipLaunchKernelGGL((select_tile_kernel<TS, XP, ANY>), grid, block, lds, stream, p);        \
+    hipLaunchKernelGGL((select_tile_kernel<TS, XP>), grid, block, lds, stream, p);        \
     return launch_status("relation_select (tile)");                                       \
   }
-  RLM_TILE_CASE(RLM_F32, float, false, false)
-  RLM_TILE_CASE(RLM_BF16, bf16, false, false)
-  RLM_TILE_CASE(RLM_F32, float, true, false)
-  RLM_TILE_CASE(RLM_BF16, bf16, true, false)
-  RLM_TILE_CASE(RLM_F32, float, false, true)
-  RLM_TILE_CASE(RLM_BF16, bf16, false, true)
-  RLM_TILE_CASE(RLM_F32, float, true, true)
-  RLM_TILE_CASE(RLM_BF16, bf16, true, true)
+  RLM_TILE_CASE(RLM_F32, float, false)
+  RLM_TILE_CASE(RLM_BF16, bf16, false)
+  RLM_TILE_CASE(RLM_F32, float, true)
+  RLM_TILE_CASE(RLM_BF16, bf16, true)
 #undef RLM_TILE_CASE
   set_error("relation_select (tile): unsupported statistics dtype %s", dtype_name(stat_dtype));
   return hipErrorInvalidValue;

@@ -153,3 +153,32 @@ def test_a_workgroup_per_query_gives_the_same_bits(device, dtype, shape, strict)
         got = relation_select_packed_seq(*select_args(row, cfg))
         torch.cuda.synchronize()
         check_same(got, [w[b:b + 1] for w in whole], (shape, b))
+
+
+@pytest.mark.parametrize("shape", [(512, 32, 64, 4, 8), (256, 64, 200, 0, 4), (128, 16, 32, 2, 8)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3e38])
+def test_scores_that_are_not_finite_whole_block_counts(device, shape, value):
+    """The shared-tile kernel at block counts that are multiples of four."""
+    test_scores_that_are_not_finite(device, shape, value)
+
+
+@pytest.mark.parametrize("context,block,slots", [(320, 64, 3), (192, 64, 4), (256, 64, 3),
+                                                 (512, 32, 4)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3e38])
+def test_multi_anchor_scores_that_are_not_finite(device, context, block, slots, value):
+    """multi_select_kernel's results, at block counts that are multiples of four and not."""
+    import dataclasses
+
+    cfg = dataclasses.replace(MULTI_CONFIGS["cfg5"], batch=2, context=context, block_size=block,
+                              local_window=64, top_blocks=4, slots=slots, k_out=5, seed=context)
+    inp = multi_selection_inputs(cfg, device=device)
+    g = torch.Generator().manual_seed(3)
+    rows = torch.randperm(context, generator=g)[: context // 8]
+    for name in ("anchor_keys", "partner_keys"):
+        inp[name][0, rows, 0, 3] = value          # one slot's element of some rows
+        inp[name][1, rows[:3]] = value            # every slot of a few rows
+        inp[name][1, rows[3:8], 1:] = value
+    got = multi_relation_select_seq(*multi_select_args(inp, cfg))
+    want = multi_relation_select_seq(*multi_select_args(upcast(inp), cfg))
+    torch.cuda.synchronize()
+    check_same(got, want, f"{context}/{block} {value}")
