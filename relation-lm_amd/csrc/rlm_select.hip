@@ -1526,6 +1526,21 @@ bool multi_tile_params(const SelectParams& p, int S, const Geometry& g, int act,
   return multi_tile_layout(tp);
 }
 
+// Whether a sequence call over a longer cache has so few candidate scores that
+// select_kernel, a workgroup per query, beats the multi-anchor tile kernel with one
+// slot (rounds of about 30 us, whatever they hold).  Tile / select_kernel, us, by
+// cache rows T, candidates and queries:
+//   T=1024  160: 256 29.3 / 16.4, 1024 29.3 / 22.6    384: 256 31.4 / 22.9, 512 30.2 / 25.5,
+//           1024 30.6 / 32.9    640: 256 33.4 / 28.1, 512 33.3 / 32.0, 768 33.4 / 37.0
+//           1024: 128 34.8 / 35.0, 512 35.1 / 40.0
+//   T=2048  160: 1024 32.3 / 29.4    384: 512 35.6 / 31.3, 768 33.0 / 35.9
+//           640: 256 39.1 / 33.5, 512 36.2 / 38.1
+//   T=4096  160: 512 38.3 / 35.8, 768 34.6 / 41.7    384: 256 37.7 / 36.4, 512 39.3 / 42.1
+bool few_queries(const Geometry& g, int candidates) {
+  const int64_t queries = g.B * g.Tq;
+  return queries <= kAloneQueries && queries * candidates <= (g.T <= 2048 ? 512 : 256) * 384;
+}
+
 // The decode form takes the latency-oriented kernel where it applies unless
 // RLM_SELECT_DECODE=0 (both kernels give identical results; the switch exists
 // to compare them).
@@ -1798,9 +1813,10 @@ hipError_t select_packed_impl(
     // the multi-anchor tile kernel with one slot, which reads the candidate
     // tiles from L2 instead of staging the cache.  B=8, T=2048, block 64, local
     // 128, top 4, K=8: 131 us, where select_kernel takes 364 us (one float64 dot
-    // per candidate per query).
+    // per candidate per query).  A few queries, whose dots are few and whose
+    // sixteens leave CUs idle, are faster on select_kernel.
     MultiTileParams mp{};
-    if (multi_tile_params(p, 1, g, act, stat, position, mp)) {
+    if (!few_queries(g, p.CAP) && multi_tile_params(p, 1, g, act, stat, position, mp)) {
       mp.single = true;
       const hipError_t me = multi_tile_launch(mp, stat, stream);
       if (me != hipSuccess || xseq == nullptr) return me;

@@ -9,6 +9,8 @@ from launched import launched
 
 from relation_lm import _native  # noqa: F401  (registers torch.ops.relation_lm)
 from relation_lm.kernels.relation_reduce import mfma_fragments, relation_reduce_fused_seq
+from relation_lm.kernels.relation_select import relation_select_packed_seq
+from relation_lm.workloads import RelationConfig, select_args, selection_inputs
 
 pytestmark = pytest.mark.gpu
 ops = torch.ops.relation_lm
@@ -76,3 +78,29 @@ def test_block_statistics_rows(device, block, rows, dtype):
     tol = eps * x64.abs().mean(2)
     assert bool(((mean.double().cpu() - want).abs() <= tol).all())
     assert bool(((std.double().cpu() - dev).abs() <= eps * dev + tol).all())
+
+
+@pytest.mark.parametrize("batch,queries,context,block,local,top,kernel", [
+    (2, 1024, 1024, 64, 128, 4, "multi_tile_kernel"),
+    (1, 512, 1024, 64, 128, 4, "::select_kernel"),       # 512 x 384 candidates
+    (3, 171, 1024, 64, 128, 4, "multi_tile_kernel"),     # 513 x 384
+    (1, 1024, 2048, 64, 32, 2, "::select_kernel"),       # 1024 x 160
+    (1, 1, 1024, 64, 128, 4, "::select_kernel"),
+    (1, 256, 4096, 64, 128, 4, "::select_kernel"),
+    (1, 257, 4096, 64, 128, 4, "multi_tile_kernel"),
+    (2, 300, 448, 64, 128, 4, "multi_tile_kernel"),      # over 256 candidates of a short cache
+    (2, 16, 448, 64, 64, 2, "select_tile_kernel")])
+def test_selection_of_few_queries(device, batch, queries, context, block, local, top, kernel):
+    """Either kernel gives the bits of the same rows in fp32, which select_kernel takes."""
+    cfg = RelationConfig("few", batch, context, 256, block, local, top, 8, BF, seed=queries)
+    inp = selection_inputs(cfg, device=device)          # the prompt's last queries
+    for name in ("anchor_query", "anchor_router_query", "partner_base"):
+        inp[name] = inp[name][:, context - queries:].contiguous()
+    inp["positions"] = inp["positions"][context - queries:].contiguous()
+    names = launched(lambda: relation_select_packed_seq(*select_args(inp, cfg)))
+    assert kernel in names, names
+    wide = {k: v.float() if v.dtype == BF else v for k, v in inp.items()}
+    got = relation_select_packed_seq(*select_args(inp, cfg))
+    want = relation_select_packed_seq(*select_args(wide, cfg))
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, w) for g, w in zip(got, want))

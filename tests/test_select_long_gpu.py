@@ -86,6 +86,25 @@ def test_positions_and_ragged_queries(device, shape):
     check(inp, none, device, f"{shape} no picks")
 
 
+@pytest.mark.parametrize("shape", [(1024, 32, 64, 4, 8), (512, 64, 128, 4, 8), (704, 64, 100, 4, 16)])
+def test_positions_and_ragged_queries_of_a_long_prompt(device, shape):
+    """The same on the shared-tile kernel, which fewer queries do not reach: 2 x 1001 of them."""
+    cfg = config(*shape, seed=79)
+    inp = selection_inputs(cfg, device="cpu")
+    g = torch.Generator().manual_seed(6)
+    rows = torch.randint(0, shape[0], (1001,), generator=g)
+    for name in ("anchor_query", "anchor_router_query", "partner_base"):
+        inp[name] = inp[name][:, rows].contiguous()
+    pos = torch.randint(0, shape[0], (2, 1001), generator=g)
+    pos[0, :8] = torch.tensor([-1, -70, 0, 1, shape[0], shape[0] + 40, shape[0] + 4000, shape[0] - 1])
+    pos[1, 960:976] = -5                   # a tile without any candidate
+    pos[1, 990:] = shape[0] + 300
+    inp["positions"] = pos.int()
+    check(inp, cfg, device, f"{shape} positions")
+    none = config(shape[0], shape[1], shape[2], 0, shape[4], seed=80)
+    check(inp, none, device, f"{shape} no picks")
+
+
 def test_equal_keys(device):
     """Every candidate ties: more members than one window, the tie rules decide."""
     cfg = config(1024, 32, 64, 4, 8, seed=9)
