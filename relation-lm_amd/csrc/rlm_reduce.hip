@@ -2689,20 +2689,22 @@ bool mlp_fits_shape(int64_t R, int64_t H, int64_t D) {
 
 template <int R, int TNB, int MODE = kMlpRaw, bool RAGGED = false>
 hipError_t launch_mlp_rt(const MlpParams& mp, hipStream_t stream) {
+  constexpr const char* what = MODE == kMlpRaw       ? "relation_hidden_linear_seq"
+                               : MODE == kMlpQueries ? "relation_mlp_reduce_seq"
+                                                     : "relation_block_seq";
   constexpr size_t lds = mlp_lds_bytes<R, TNB, MODE>();
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(&relation_mlp_kernel<R, TNB, MODE, RAGGED>),
       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   if (attr != hipSuccess) {
-    set_error("relation_hidden_linear_seq: cannot reserve %zu bytes of LDS: %s", lds,
-              hipGetErrorString(attr));
+    set_error("%s: cannot reserve %zu bytes of LDS: %s", what, lds, hipGetErrorString(attr));
     return attr;
   }
   const int rows = MODE == kMlpQueries ? mp.tile_rows : kMlpRows;
   const int64_t tiles = (mp.h.rows + rows - 1) / rows;
   hipLaunchKernelGGL((relation_mlp_kernel<R, TNB, MODE, RAGGED>), dim3(static_cast<unsigned>(tiles)),
                      dim3(kMlpThreads), lds, stream, mp);
-  return launch_status("relation_hidden_linear_seq");
+  return launch_status(what);
 }
 
 template <int R, int MODE>
@@ -3659,7 +3661,8 @@ extern "C" hipError_t rlm_relation_mlp_reduce_seq(
   hipLaunchKernelGGL(mfma_fragments2_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)),
                      dim3(256), 0, stream, static_cast<const uint16_t*>(product_weight->data), H, R,
                      static_cast<const uint16_t*>(second_weight->data), frag ? 0 : D, H, frags);
-  RLM_REQUIRE(launch_status(what) == hipSuccess, "%s: packing launch failed", what);
+  const hipError_t pe = launch_status(what);
+  if (pe != hipSuccess) return pe;
   HiddenParams& p = mp.h;
   p.B = B;
   p.Tq = Tq;

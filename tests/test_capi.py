@@ -355,3 +355,34 @@ def test_fused_reduce_fits_from_python():
     assert not relation_reduce_fused_seq_fits(e, o, pi, wm, torch.empty(576, 512, dtype=bf))
     assert not relation_reduce_fused_seq_fits(e, o.float(), pi, wm,
                                               torch.empty(512, 512, dtype=bf))
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0,
+                    reason="valid descriptors of made-up addresses: only where nothing can launch")
+def test_launch_failures_carry_the_called_name(lib):
+    """Without a device every launch fails: the message names the entry point that was called,
+    and the status is the runtime's own."""
+    b, t, r, h, d, k, s = 1, 64, 64, 128, 256, 4, 2
+    vec = tensor([d])
+    caches = [tensor([b, t, 2 * h], RLM_BF16), tensor([b, t, r], RLM_BF16)]
+    frags = [tensor([h // 32, r // 16, 64, 8], RLM_BF16), tensor([d // 32, h // 16, 64, 8], RLM_BF16)]
+    refs = lambda *ts: [ctypes.byref(x) for x in ts]  # noqa: E731
+    calls = {
+        "rlm_relation_hidden_linear_seq": refs(
+            *caches, tensor([b, t], RLM_I32), tensor([b, t, k], RLM_I32), *frags,
+            tensor([b, t, k, d])),
+        "rlm_relation_mlp_reduce_seq": refs(
+            *caches, tensor([b, t], RLM_I32), tensor([b, t, k], RLM_I32), tensor([h, r], RLM_BF16),
+            tensor([d, h], RLM_BF16), vec, tensor([b, t, k]), vec, vec, tensor([t], RLM_I64))
+        + [ctypes.c_double(1e-5)] + refs(tensor([h * r + d * h], RLM_BF16), tensor([b, t, d])),
+        "rlm_relation_block_seq": refs(
+            *caches, tensor([b, t * s], RLM_I32), tensor([b, t * s, k], RLM_I32), *frags, vec,
+            tensor([b, t, s, k]), vec, vec, tensor([s]), tensor([]), tensor([b, t, d], RLM_BF16),
+            tensor([t], RLM_I64))
+        + [ctypes.c_double(1e-5)] + refs(tensor([1 << 20]), tensor([b, t, d], RLM_BF16)) + [None],
+    }
+    for name, args in calls.items():
+        status = getattr(lib, name)(*args, ctypes.c_void_p(0))
+        message = lib.rlm_last_error().decode()
+        assert status not in (0, HIP_ERROR_INVALID_VALUE), (name, status, message)
+        assert message.startswith(name[4:] + ":"), (name, message)
