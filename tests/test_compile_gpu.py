@@ -336,3 +336,16 @@ def test_opcheck_every_registered_op(device):
         print(f"opcheck {name}", flush=True)
         result = torch.library.opcheck(op, args)
         assert all(v == "SUCCESS" for v in result.values()), (name, result)
+
+
+def test_no_operator_outside_the_sweeps():
+    """Every operator of the library's namespaces is in the sweep above or, a step of the block
+    module, in tests/test_relation_block_gpu.py's."""
+    registered = {n for n in torch._C._dispatch_get_all_op_names()
+                  if n.startswith(("relation_lm", "relationlex"))}
+    assert {n.split("::")[0] for n in registered} == {"relation_lm", "relationlex",
+                                                      "relation_lm_block"}
+    assert {n for n in registered if n.startswith("relation_lm_block::")} == {
+        "relation_lm_block::relation_block_seq_out"}
+    assert {n.split("::")[1] for n in registered
+            if not n.startswith("relation_lm_block::")} == set(OP_NAMES)
