@@ -548,13 +548,15 @@ hipError_t rlm_relation_reduce_fused_seq(
 
 /*
  * Whether rlm_relation_reduce_fused_seq takes these operands (no reference
- * counterpart: the capability query behind relation_lm::relation_reduce_fused_seq,
- * which runs the unfused relation_hidden_cached_seq -> relation_linear ->
- * relation_norm_reduce_seq chain for every other shape, e.g. the reference's
- * fp32 D = 576 cases of tests/test_relation_reduce_gpu.py:163-200).  Returns 1
- * for bf16 caches and weights, 1 <= K <= 16, R in {32,64,128}, H a multiple of
- * 128, D in {128, 256, 384, 512} and 16-byte aligned operand_cache,
- * product_weight and second_weight; 0 otherwise.  Reads descriptors only.
+ * counterpart).  Returns 1 for bf16 caches and weights, 1 <= K <= 16, R in
+ * {32,64,128}, H a multiple of 128, D in {128, 256, 384, 512} and 16-byte aligned
+ * operand_cache, product_weight and second_weight (either form); 0 otherwise.
+ * relation_lm::relation_reduce_fused_seq takes a second_weight in fragment order
+ * exactly where this is 1; which kernel it runs (this one,
+ * rlm_relation_mlp_reduce_seq, or the relation_hidden_cached_seq ->
+ * relation_linear -> relation_norm_reduce_seq chain, e.g. for the reference's fp32
+ * D = 576 cases of tests/test_relation_reduce_gpu.py:163-200) also depends on the
+ * number of rows.  Reads descriptors only.
  */
 int rlm_relation_reduce_fused_seq_fits(const rlm_tensor* expanded_cache,
                                        const rlm_tensor* operand_cache,

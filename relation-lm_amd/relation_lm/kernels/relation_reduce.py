@@ -343,9 +343,12 @@ def relation_reduce_fused_seq_fits(
     product_weight: Tensor,
     second_weight: Tensor,
 ) -> bool:
-    """True when ``relation_reduce_fused_seq`` runs these operands as one fused kernel, False
-    when it runs the three-launch chain instead (fp32, d_model 576, K > 16, ...).  Reads only
-    shapes, dtypes and pointer alignment; launches nothing."""
+    """True when ``relation_reduce_fused_seq`` takes these operands with ``second_weight`` in
+    either form, row-major or MFMA fragment order: bf16, 1 <= K <= 16, relation dim 32, 64 or
+    128, hidden dim a multiple of 128, d_model 128, 256, 384 or 512, 16-byte aligned.  False
+    when it needs the [D, H] weight (fp32, d_model 576, K > 16, ...).  It does not tell which
+    kernel runs: that also depends on the number of queries.  Reads only shapes, dtypes and
+    pointer alignment; launches nothing."""
     lib = _native.c_library()
     return bool(lib.rlm_relation_reduce_fused_seq_fits(
         *(ctypes.byref(_desc(t)) for t in (expanded_cache, operand_cache, partner_index,
@@ -366,15 +369,19 @@ def relation_reduce_fused_seq(
     positions: Tensor,
     norm_eps: float,
 ) -> Tensor:
-    """Relation hidden -> second linear -> norm-reduce in one kernel -> f32 [B, Tq, D].
+    """Relation hidden -> second linear -> norm-reduce in one call -> f32 [B, Tq, D].
 
     Same result as ``relation_norm_reduce_seq(relation_linear(relation_hidden_cached_seq(...),
     second_weight, second_bias), ...)`` (the reference's three-call sequence,
     benchmarks/benchmark_relation_reduce.py:55-64) with bf16 caches and weights: the
     hidden is rounded to bf16 before the second linear, as the unfused bf16 linear does.
-    Operands the fused kernel does not take (fp32, d_model outside {128, 256, 384,
-    512}, K > 16, ...) run that three-op chain on HIP instead, so every shape the
-    reference's ops accept goes through this op.
+    With bf16 operands, K <= 16 and a hidden dim that is a multiple of 128 it is one of two
+    kernels that keep the hidden and the raw rows on chip: 128-row tiles (d_model 128, 256, 384
+    or 512) or 64-row tiles (any d_model that is a multiple of 32 up to 768, from 1536 relation
+    rows on; a launch of the same call packs its weights), whichever is faster where both take
+    the shape.  Other operands (fp32, K > 16, fewer rows at other d_model, ...) run the
+    three-op chain on HIP, so every shape the reference's ops accept goes through this op.
+    ``second_weight`` may be in MFMA fragment order where ``relation_reduce_fused_seq_fits``.
     """
     return torch.ops.relation_lm.relation_reduce_fused_seq(
         expanded_cache, operand_cache, anchor_index, partner_index, product_weight,
