@@ -109,3 +109,14 @@ def test_zero_weight_rows_do_not_count(device):
     torch.cuda.synchronize()
     assert bool(torch.isfinite(got).all()) and torch.equal(got, base)
     assert want.shape == got.shape
+
+
+def test_long_calls_equal_their_batch_rows(device):
+    """A hidden of 2.4 GB, which never exists: the call's bits are those of its batch rows."""
+    red, expanded, a, p, score, pos = inputs(device, 8, 2048, 8, 64, 4608, 128, rows=512)
+    got = fused(red, expanded, a, p, score, pos)
+    for b in range(8):
+        one = dict(red, operand_cache=red["operand_cache"][b:b + 1])
+        want = fused(one, expanded[b:b + 1], a[b:b + 1], p[b:b + 1], score[b:b + 1], pos)
+        torch.cuda.synchronize()
+        assert torch.equal(got[b:b + 1], want), b
