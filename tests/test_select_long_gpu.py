@@ -2,7 +2,8 @@
 
 relation_select_packed_seq with bf16 activations takes a matrix-core-filtered kernel
 for every cache of at most 64 blocks: rlm_select_tile.hip up to 512 rows and 256
-candidates, rlm_multi_tile.hip (one slot) beyond.  The same call in fp32 runs
+candidates, rlm_multi_tile.hip (one slot) beyond, except for few queries there, which
+take select_kernel too.  The same call in fp32 runs
 select_kernel (rlm_select.hip), one float64 dot per candidate; on the same values both
 must give the same bits -- indices, scores, sentinels -- also for infinite, NaN and
 overflowing scores, where the filter's error bound does not hold.
